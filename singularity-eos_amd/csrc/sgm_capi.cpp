@@ -362,7 +362,8 @@ int sgm_set_Vinet(sgm_ctx *ctx, int m, double rho0, double T0, double B0, double
   }
   EosDev e{};
   e.kind = KIND_VINET;
-  const double p[12] = {rho0, T0, B0, BP0, A0, Cv0, E0, S0, VIP[1],
+  const double p[12] = {rho0, T0, B0, 9.0 * robust::ratio(B0, VIP[1] * VIP[1] * rho0), A0, Cv0,
+                        E0, robust::ratio(T0, rho0), VIP[1],
                         pmath::cbrt(10 * robust::EPS()) * rho0, VIP[2], VIP[3]};
   for (int i = 0; i < 12; ++i) e.m.p[i] = p[i];
   e.nvinet_skip = nskip;

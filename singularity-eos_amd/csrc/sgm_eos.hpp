@@ -55,7 +55,8 @@ struct TableDev {
 //  IdealGas  {Cv, gm1}
 //  StiffGas  {Cv, gm1, Pinf, qq}
 //  Gruneisen {C0, s1, s2, s3, G0, b, rho0, T0, P0, Cv, rho_max}
-//  Vinet     {rho0, T0, B0, BP0, A0, Cv0, E0, S0, VIP1, min_density, VIP2, VIP3}
+//  Vinet     {rho0, T0, B0, 9 B0 / (VIP1^2 rho0), A0, Cv0, E0, T0 / rho0, VIP1,
+//             min_density, VIP2, VIP3}
 // Vinet Horner coefficients (d2..d40 then VIP0..VIP42) live in `coef`;
 // nvinet_skip counts the leading Horner steps that can be skipped because
 // every coefficient they touch is exactly zero (the sums stay exactly 0
@@ -541,7 +542,8 @@ SGM_NOINL void rhoe_PT(const Real *p, Real P, Real T, Real &rho, Real &sie, int 
 } // namespace grun
 
 namespace vinet { // singularity-eos/eos/eos_vinet.hpp:228-352
-// p = {rho0, T0, B0, BP0, A0, Cv0, E0, S0, VIP1, min_density}; coef = d2..d40 (39) then
+// p = {rho0, T0, B0, 9 B0 / (VIP1^2 rho0), A0, Cv0, E0, T0 / rho0, VIP1, min_density, ...}
+// (the two quotients of constants rounded as the formula rounds them); coef = d2..d40 (39) then
 // VIP[0..42] (43). Returns energy and pressure (and optionally the sound speed^2 term).
 struct EP {
   Real e, P, cs2;
@@ -569,9 +571,8 @@ SGM_HD EP F_DT(const Real *p, const Real *coef, int nskip, Real rho, Real T) {
   sumP = 1.0 + sumP * (onemx * onemx);
   sumB = sumB * onemx;
   sumE = VIP1 * onemx * sumE;
-  Real energy = 9.0 * robust::ratio(B0, VIP1 * VIP1 * rho0) *
-                    (p[10] - expetatimes1mx * (p[10] - sumE)) -
-                (A0 * B0) * (robust::ratio(T0, rho0) - robust::ratio(T0, rho));
+  Real energy = p[3] * (p[10] - expetatimes1mx * (p[10] - sumE)) -
+                (A0 * B0) * (p[7] - robust::ratio(T0, rho));
   Real pressure = 3.0 * B0 * x2inv * onemx * expetatimes1mx * sumP;
   EP out;
   out.cs2 = 0;

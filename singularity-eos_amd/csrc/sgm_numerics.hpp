@@ -50,13 +50,24 @@ constexpr double scale_up = 4503599627370496.0;
 constexpr std::int64_t mantissa_mask = (std::int64_t(1) << 52) - 1;
 constexpr std::int64_t low_mask = (std::int64_t(1) << 26) - 1;
 
+// d / 3 for 0 <= d < 2^52 in two 26-bit digits: a 64-bit division by a
+// constant costs a 64 x 64 high product, these two 32-bit ones
+// (the table's log: 253 -> 221 cycles on one wave)
+SGM_HD std::int64_t div3(std::int64_t d) {
+  const std::uint32_t dh = (std::uint32_t)(d >> 26), dl = (std::uint32_t)(d & low_mask);
+  const std::uint32_t qh = dh / 3u;
+  const std::uint32_t rest = ((dh - 3u * qh) << 26) | dl;  // < 3 * 2^26
+  return ((std::int64_t)qh << 26) + rest / 3u;
+}
 SGM_HD double lg(double x) {
   const std::int64_t xi = as_int(x) - one_as_int;
   const std::int64_t fr = xi & mantissa_mask;
-  const std::int64_t hi = fr >> 26;
-  const std::int64_t lo = fr & low_mask;
-  const std::int64_t sq = hi * hi + ((hi * lo) >> 25);
-  return static_cast<double>(xi + ((fr - sq) / 3)) * scale_down;
+  const std::uint32_t hi = (std::uint32_t)(fr >> 26);
+  const std::uint32_t lo = (std::uint32_t)(fr & low_mask);
+  // fr - fr^2 / 2^52, never negative: the square is taken by its floor
+  const std::int64_t sq =
+      (std::int64_t)((std::uint64_t)hi * hi + (((std::uint64_t)hi * lo) >> 25));
+  return static_cast<double>(xi + div3(fr - sq)) * scale_down;
 }
 SGM_HD double pow2(double x) {
   const std::int64_t xi = static_cast<std::int64_t>(x * scale_up);
@@ -281,6 +292,19 @@ SGM_HD bool find_root(const F &f, Real ytarget, Real xguess, Real xmin, Real xma
 // Both are within a few ulp of the correctly rounded values.
 // ---------------------------------------------------------------------------
 namespace pmath {
+// x / 3, correctly rounded, for x normal and far from the range's ends: a
+// product with the rounded reciprocal (within one ulp) and one residual
+// correction (Markstein) instead of the general division's scaling,
+// reciprocal and refinement: cbrt's five steps 1072 -> 775 cycles on one wave
+SGM_HD double div3(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double third = 1.0 / 3.0;
+  const double q = x * third;
+  return __builtin_fma(__builtin_fma(-3.0, q, x), third, q);
+#else
+  return x / 3.0;
+#endif
+}
 SGM_HD double pow2i(int k) { // 2^k for -1022 <= k <= 1023
   return nqt::as_double(static_cast<std::int64_t>(k + 1023) << 52);
 }
@@ -336,7 +360,7 @@ SGM_HD double cbrt(double x) {
   const double mm = s == 0 ? m : (s == 1 ? 2.0 * m : 4.0 * m); // [1, 8)
   double y = (-0.011593381976926909 * mm + 0.23742467276201396) * mm + 0.8208312163657417;
 #pragma unroll
-  for (int i = 0; i < 5; ++i) y = (2.0 * y + mm / (y * y)) / 3.0;
+  for (int i = 0; i < 5; ++i) y = div3(2.0 * y + mm / (y * y));
   y *= pow2i(q + adj);
   return x < 0 ? -y : y;
 }
