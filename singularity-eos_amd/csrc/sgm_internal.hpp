@@ -30,6 +30,22 @@ struct VinetHost {
   Real *d_coef = nullptr;
 };
 
+// Work arrays, fork streams and events of one batched closure call
+// (sgm_batch.hip): one call at a time in stream order, `done` marking the
+// last one's end.
+struct BatchWs {
+  void *buf = nullptr;
+  size_t bytes = 0;
+  hipStream_t aux[5] = {};
+  hipEvent_t ev[6] = {};
+  hipEvent_t done = nullptr;
+  hipStream_t last = nullptr;
+  unsigned long long used = 0;
+  void release();
+};
+// cells of one batch (longer calls run as several): 0.8 GB of work arrays
+constexpr long BATCH_MAX_CELLS = 1L << 20;
+
 } // namespace sgm
 
 struct sgm_ctx {
@@ -52,6 +68,10 @@ struct sgm_ctx {
   size_t drv_cells_bytes = 0, drv_entries_bytes = 0;
   long drv_plan_builds = 0, drv_plan_reuses = 0;  // calls that built / reused the plan
   std::mutex drv_mu;
+  // workspaces of batched closure calls: at most this many overlap
+  sgm::BatchWs batch[4];
+  unsigned long long batch_clock = 0;
+  std::mutex batch_mu;
 };
 
 namespace sgm {
@@ -77,6 +97,12 @@ inline unsigned long long ctx_mod_mask(const sgm_ctx *ctx) {
     if (ctx->host_eos[i].mods) m |= 1ull << i;
   return m;
 }
+// A closure call over a's cells as one batch of the binned kernels; taken =
+// false when the call has to go to the plain kernel (its stream is being
+// captured, or there is no memory for the work arrays).
+hipError_t launch_pte_batch(sgm_ctx *ctx, int method, const PteArgs &a, const MixParamsDev &P,
+                            hipStream_t s, bool &taken);
+int batch_cells_per_wave(long ncell, int ncu);
 // MixParams as the kernels take them (NULL = the reference's defaults)
 MixParamsDev to_dev(const sgm_mix_params *p);
 // A batched plan over a CSR topology (sgm_plan_create) whose cells with fewer

@@ -48,11 +48,14 @@ struct ParkArgs {
   int stride = 0;                   // FP64 words per record
   double *rec = nullptr;            // records
   int *cell_of = nullptr;           // cell id per record
-  const int *run_of = nullptr;      // per bin position: signature run
+  // per bin position: signature run (null: the bin is one run, 0)
+  const int *run_of = nullptr;
   const int *run_base = nullptr;    // per run: first record
   const int *run_cap = nullptr;     // per run: records available
   int *run_count = nullptr;         // per run: records claimed (claims past cap are not parked)
-  const int *wave_run = nullptr;    // per tail wave: its run
+  // per tail wave: its run (null, with wave_first: one run, wave w on the
+  // records of its w-th slot; nwaves is then an upper bound)
+  const int *wave_run = nullptr;
   const int *wave_first = nullptr;  // per tail wave: its first record within the run
   int nwaves = 0;
   // the tail's second level: a cell still iterating `after2` iterations into

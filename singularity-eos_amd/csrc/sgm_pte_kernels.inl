@@ -250,7 +250,9 @@ __attribute__((amdgpu_waves_per_eu(SGM_BIN_WAVES_PER_EU,
   }
   const int lane = threadIdx.x & 63;
   const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  if (chunk < 64) chunk = 64;  // one claim must cover a whole wave
+  // a claim covers every lane that takes cells: fewer than 64 cells per claim
+  // keep the lanes past them idle (small batches, spread over more waves)
+  if (chunk < 1) chunk = 1;
   SysOf<NM, METHOD, false> s;
   DriverState d;
   CellStatus st;
@@ -258,7 +260,7 @@ __attribute__((amdgpu_waves_per_eu(SGM_BIN_WAVES_PER_EU,
   int off = 0;
   bool park_ok = false;  // this lane may still park its cell (one attempt per cell)
   bool active = false;  // this lane holds a cell that is still iterating
-  bool done = false;    // the bin is exhausted for this wave
+  bool done = lane >= chunk;  // the bin is exhausted for this lane
   long rbase = 0, rend = 0;  // wave-uniform reserve [rbase, rend) of bin positions
   for (;;) {
     // hand out cells to idle lanes (REFILL_BATCH at a time)
@@ -316,7 +318,7 @@ __attribute__((amdgpu_waves_per_eu(SGM_BIN_WAVES_PER_EU,
     } else if (active && park_ok && d.niter >= pk.after) {
       // a straggler: save it in its signature run's records for the tail
       // kernel and free the lane
-      const int r = pk.run_of[jpos];
+      const int r = pk.run_of ? pk.run_of[jpos] : 0;
       const int i = atomicAdd(pk.run_count + r, 1);
       if (i < pk.run_cap[r]) {
         const long slot = (long)pk.run_base[r] + i;
@@ -373,18 +375,22 @@ __device__ __forceinline__ void tail_wide(const PteArgs &a, const MixParamsDev &
   constexpr int per_slot = 64 / TailGroup(PTE_RHOT, NM);
   constexpr int PW = ParkWordCount<Sys>();
   __shared__ double probe_lds[PW];
-  const long items = (long)pk.nwaves * per_slot;
+  // one run: its claimed records are the first ones, in claim order
+  const int claimed = min(pk.run_count[0], pk.run_cap[0]);
+  const long items = pk.wave_run ? (long)pk.nwaves * per_slot : claimed;
   // these waves carry the bin's longest dependency chains: let them issue
   // ahead of other kernels' waves on their CU
   __builtin_amdgcn_s_setprio(3);
   for (;;) {
     const int item = __builtin_amdgcn_readfirstlane(atomicAdd(pk.l2_next, lane == 0 ? 1 : 0));
     if (item >= items) break;
-    const int w = item / per_slot;
-    const int r = pk.wave_run[w];
-    const int nr = min(pk.run_count[r], pk.run_cap[r]);
-    const int i = pk.wave_first[w] + item % per_slot;
-    if (i >= nr) continue;
+    int r = 0, i = item;
+    if (pk.wave_run) {
+      const int w = item / per_slot;
+      r = pk.wave_run[w];
+      i = pk.wave_first[w] + item % per_slot;
+      if (i >= min(pk.run_count[r], pk.run_cap[r])) continue;
+    }
     const long slot = (long)pk.run_base[r] + i;
     const long c = pk.cell_of[slot];
     if (c < 0) continue;  // finished in level 1
@@ -437,13 +443,29 @@ __attribute__((amdgpu_waves_per_eu(WPE, WPE))) pte_tail_kernel(PteArgs a, MixPar
     const int lpc = grp ? G : 1;  // lanes per cell
     const int spb = grp ? 1 : G;  // wave slots per block step
     const int g = lane % lpc, base = lane - g;
-    for (long W = blockIdx.x; W * spb < pk.nwaves; W += gridDim.x) {
-      const long w = grp ? W : W * G + lane / per_slot;
-      if (w >= pk.nwaves) continue;
-      const int r = pk.wave_run[w];
-      const int nr = min(pk.run_count[r], pk.run_cap[r]);
-      const int i = pk.wave_first[w] + (grp ? lane / G : lane % per_slot);
-      if (i >= nr) continue;  // in a group, the whole group skips
+    // one run: a lane per cell is spread over the whole grid first, so that a
+    // wave runs as few cells (each with root finds of its own length) as the
+    // population allows
+    const bool one_run = !pk.wave_run;
+    const int claimed = one_run ? min(pk.run_count[0], pk.run_cap[0]) : 0;
+    const int lpw = one_run && !grp
+                        ? min(64, max(1, (claimed + (int)gridDim.x - 1) / (int)gridDim.x))
+                        : per_slot;
+    const long steps = !one_run ? (pk.nwaves + spb - 1) / spb : (claimed + lpw - 1) / lpw;
+    for (long W = blockIdx.x; W < steps; W += gridDim.x) {
+      int r = 0, i;
+      if (one_run) {
+        const int k = grp ? lane / G : lane;
+        i = (int)W * lpw + k;
+        if (k >= lpw || i >= claimed) continue;
+      } else {
+        const long w = grp ? W : W * G + lane / per_slot;
+        if (w >= pk.nwaves) continue;
+        r = pk.wave_run[w];
+        i = pk.wave_first[w] + (grp ? lane / G : lane % per_slot);
+        // in a group, the whole group skips
+        if (i >= min(pk.run_count[r], pk.run_cap[r])) continue;
+      }
       const long slot = (long)pk.run_base[r] + i;
       const long c = pk.cell_of[slot];
       if (c < 0) continue;  // finished in level 1
@@ -560,7 +582,7 @@ hipError_t tail_launch(int nm, const PteArgs &a, const MixParamsDev &P, const Pa
   const int ncu = device_cu_count();
   const int cap = (nm >= 5 ? SGM_TAIL_WAVES_PER_EU_LARGE : 2) * 4 * ncu;
   const int G = TailGroup(METHOD, nm);
-  const int g1 = (pk.nwaves + G - 1) / G;
+  const int g1 = pk.wave_run ? (pk.nwaves + G - 1) / G : pk.nwaves * (64 / G);
   const int g = g1 < cap ? g1 : cap;
   const bool l2 = G > 1 && pk.after2 > 0 && pk.l2_count &&
                   P.line_search_max_iter <= G && (!TailWide(METHOD, nm) || pk.l2_next);

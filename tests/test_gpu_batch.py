@@ -1,0 +1,127 @@
+"""The two routes of a plain closure call: the batch (cells sorted on the
+device, binned kernels with parking and tails, work arrays of the context)
+that calls with more than two materials per cell on average take, and the
+plain kernels, which the same call takes while its stream is being captured.
+Same cells, same bits, at the sizes where the batch changes its lanes per
+wave, with pure, malformed and modified cells among them, and from several
+streams at once (more than the context has workspaces)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+FIELDS = ("rho", "vfrac", "sie", "temp", "press")
+
+
+def cells(workloads, ctx, n, seed, pure=True):
+    """Uneven cells; every 11th reduced to its first material and, past 60,
+    one cell naming a material outside the registry."""
+    a = workloads.uneven(ctx, n, seed=seed)
+    off = a["offsets"].astype(np.int64)
+    keep = np.ones(a["nnz"], dtype=bool)
+    if pure:
+        for c in range(5, n, 11):
+            keep[off[c] + 1:off[c + 1]] = False
+    cnt = np.add.reduceat(keep, off[:-1])
+    for k in FIELDS:
+        a[k] = a[k][keep].copy()
+    a["mat_ids"] = a["mat_ids"][keep].copy()
+    a["offsets"] = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32)
+    a["nnz"] = int(keep.sum())
+    if n > 60:
+        a["mat_ids"][a["offsets"][60]] = 60
+    return a
+
+
+def cell_input(a, method):
+    first = a["offsets"][:-1]
+    if method == 2:
+        return a["temp"][first].copy()
+    if method == 3:
+        return np.abs(a["press"][first]) + 1e5
+    return a["sie_tot"]
+
+
+class Call:
+    def __init__(self, torch, sgm, a, method, tight):
+        self.torch, self.method, self.n, self.nnz = torch, method, a["ncell"], a["nnz"]
+        self.base = {k: torch.tensor(a[k], device="cuda") for k in FIELDS}
+        self.w = {k: v.clone() for k, v in self.base.items()}
+        self.off = torch.tensor(a["offsets"], device="cuda")
+        self.mat = torch.tensor(a["mat_ids"], device="cuda")
+        self.vt = torch.tensor(a["vfrac_tot"], device="cuda")
+        self.cin = torch.tensor(cell_input(a, method), device="cuda")
+        self.st = {k: torch.full((self.n,), -1, dtype=torch.int32, device="cuda")
+                   for k in ("conv", "niter", "err")}
+        self.resid = torch.zeros(self.n, dtype=torch.float64, device="cuda")
+        self.params = sgm.mix_params(tight=tight)
+
+    def run(self, ctx, stream):
+        for k in FIELDS:
+            self.w[k].copy_(self.base[k])
+        rc = ctx.pte(self.method, self.n, self.nnz, self.off, self.mat, self.w["rho"],
+                     self.w["vfrac"], self.w["sie"], self.w["temp"], self.w["press"], self.vt,
+                     self.cin, params=self.params, resid=self.resid, stream=stream, **self.st)
+        assert rc == 0
+
+    def result(self):
+        return {k: v.cpu().numpy().copy()
+                for k, v in dict(self.w, **self.st, resid=self.resid).items()}
+
+
+def same(x, y):
+    return all(np.array_equal(x[k], y[k], equal_nan=x[k].dtype.kind == "f") for k in x)
+
+
+def captured(torch, ctx, call):
+    """The call's plain kernels: recorded into a graph, replayed twice."""
+    g = torch.cuda.CUDAGraph()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        with torch.cuda.graph(g, stream=s):
+            call.run(ctx, s.cuda_stream)
+    got = []
+    for _ in range(2):
+        g.replay()
+        torch.cuda.synchronize()
+        got.append(call.result())
+    assert same(*got)
+    return got[0]
+
+
+@pytest.mark.parametrize("method,n", [(0, 1), (0, 5), (0, 64), (0, 65), (0, 4097), (0, 20000),
+                                      (1, 300), (2, 1500), (3, 300), (4, 200)])
+def test_batch_matches_plain_kernels(sgm, workloads, torch_gpu, method, n):
+    torch = torch_gpu
+    ctx, _ = workloads.pool_context()
+    if n == 1500:
+        ctx.set_modifiers(4, shifted=True, shift=1e8)
+    a = cells(workloads, ctx, n, 0x5EED0000 + 900 + n + method, pure=n > 5)
+    assert a["nnz"] > 2 * n
+    call = Call(torch, sgm, a, method, tight=method == 0)
+    call.run(ctx, 0)
+    torch.cuda.synchronize()
+    batch = call.result()
+    assert same(batch, captured(torch, ctx, call))
+    ctx.close()
+
+
+def test_batches_from_several_streams(sgm, workloads, torch_gpu):
+    torch = torch_gpu
+    ctx, _ = workloads.pool_context()
+    calls = [Call(torch, sgm, cells(workloads, ctx, n, 0x5EED0000 + 950 + i), 0, False)
+             for i, n in enumerate((900, 3000, 200, 2500, 1200, 5000, 777))]
+    want = []
+    for c in calls:
+        c.run(ctx, 0)
+        torch.cuda.synchronize()
+        want.append(c.result())
+    streams = [torch.cuda.Stream() for _ in calls]
+    for _ in range(3):
+        for c, s in zip(calls, streams):
+            with torch.cuda.stream(s):
+                c.run(ctx, s.cuda_stream)
+        torch.cuda.synchronize()
+        for c, w in zip(calls, want):
+            assert same(c.result(), w)
+    ctx.close()
