@@ -52,6 +52,35 @@ def test_forward_matches_fp64_reference(torch_gpu, L, ref):
     mlp.close()
 
 
+@pytest.mark.parametrize("B", [1, 15, 16, 17, 63, 65, 129, 16385])
+def test_row_tiles_match_fp64_reference(torch_gpu, L, ref, B):
+    """Partial waves and tiles, and (16,385 rows: 257 tiles) blocks that take a
+    second tile: outputs and gradients against the FP64 network."""
+    torch = torch_gpu
+    mlp = L.MLP(seed=5)
+    n = min(B, 300)
+    X, Xr, T = random_batch(torch, ref, n, 3)
+    tgt = torch.tensor(T, device="cuda")
+    idx = torch.arange(B, dtype=torch.int32, device="cuda") % n
+    Y = mlp.forward(torch, X, idx).cpu().numpy()
+    Yr, _ = ref.forward(mlp.params(), Xr)
+    rows = idx.cpu().numpy()
+    # bf16 activations (2^-9 each) through four layers
+    assert np.abs(Y[:, :7] - Yr[rows][:, :7]).max() < 0.05 * max(1.0, np.abs(Yr[:, :7]).max())
+    g, loss = mlp.gradients(torch, X, tgt, idx)
+    g = g.cpu().numpy().astype(np.float64)
+    cnt = np.bincount(rows, minlength=n).astype(float)
+    # the batch's gradient: the reference's rows weighted by their count
+    gr = np.zeros(ref.NPARAM)
+    for k in np.unique(cnt):
+        sel = cnt == k
+        gk, _ = ref.gradients(mlp.params(), Xr[sel], T[sel])
+        gr += gk * sel.sum() * k / B
+    # bf16 gradients into the products: 2^-9 per element
+    assert np.linalg.norm(g - gr) < 0.03 * np.linalg.norm(gr)
+    mlp.close()
+
+
 def test_gradients_match_fp64_reference(torch_gpu, L, ref):
     torch = torch_gpu
     mlp = L.MLP(seed=4)
