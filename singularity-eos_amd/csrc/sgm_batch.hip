@@ -2,8 +2,8 @@
 // sorted by material count and signature on the device and solved by the
 // batched kernels (register-resident bins with straggler parking, tails),
 // bin bounds and record bases read on the device, so nothing comes back to
-// the host. The work arrays and fork streams come from the context's batch
-// workspaces. What bounds a plain call over uneven cells is its slowest
+// the host. The work arrays come from the context's batch workspaces, or from
+// the caller (the server's arena). What bounds a plain call over uneven cells is its slowest
 // cell's chain of Newton passes: the plain kernel runs it on one lane, behind
 // the wave's cells of other material counts and through every repeat of a
 // fixed point. 20,011 uneven cells, RhoT at 1e-10: 91 -> 12.2 ms; 1,000
@@ -17,17 +17,15 @@
 namespace sgm {
 namespace {
 
-// bins: material counts 2..6; per bin of `small`: {run base, run capacity,
-// run count, level-2 count, level-2 queue, cell counter}
-constexpr int NBIN = 5, NSMALL = 6;
+constexpr int NBIN = 5, NSMALL = BATCH_SMALL;  // bins: material counts 2..6
 constexpr int BATCH_PARK_AFTER = 20, BATCH_AFTER2 = 4;  // as plans
 
 // From the sorted keys: per material count 2..6 {start, count} and the bin's
-// record table (one run per bin, a record for each of its cells at the cells'
-// own positions); range 0 the cells before them (fewer than 2 materials),
+// record table (one run per bin: nrec records, or, with nrec 0, a record for
+// each of its cells at the cells' own positions); range 0 the cells before them (fewer than 2 materials),
 // range 6 those past the register-resident counts.
 __global__ void batch_tables_kernel(const unsigned long long *__restrict__ keys, long n,
-                                    int max_nm, long *__restrict__ range,
+                                    int max_nm, int nrec, long *__restrict__ range,
                                     int *__restrict__ small) {
   __shared__ long pos[NBIN + 1];  // first position with a count of at least k + 2
   const int t = threadIdx.x;
@@ -49,8 +47,8 @@ __global__ void batch_tables_kernel(const unsigned long long *__restrict__ keys,
     range[2 * (t + 1)] = start;
     range[2 * (t + 1) + 1] = count;
     int *s = small + NSMALL * t;
-    s[0] = (int)start;
-    s[1] = (int)count;
+    s[0] = nrec ? t * nrec : (int)start;
+    s[1] = nrec ? nrec : (int)count;
     s[2] = s[3] = s[4] = s[5] = 0;
   } else if (t == NBIN) {
     range[0] = 0;
@@ -60,10 +58,20 @@ __global__ void batch_tables_kernel(const unsigned long long *__restrict__ keys,
   }
 }
 
+// Lanes of a wave that take cells: all 64 once the batch fills four waves per
+// CU with them, fewer below, where waves are plentiful and each pass of a
+// wave costs the sum of its lanes' material kinds.
+int cells_per_wave(long ncell, int ncu) {
+  int c = 64;
+  while (c > 4 && ncell < 4L * ncu * c) c /= 2;
+  return c;
+}
+
 struct Layout {
   size_t keys, keys2, ids, sorted, range, small, cell_of, rec, tmp, tmp_bytes, total;
 };
-hipError_t layout(int method, long n, Layout &L) {
+// nrec: straggler records per bin; 0: one per cell
+hipError_t layout(int method, long n, int nrec, Layout &L) {
   size_t o = 0;
   auto take = [&](size_t b) {
     const size_t at = o;
@@ -76,8 +84,9 @@ hipError_t layout(int method, long n, Layout &L) {
   L.sorted = take(4 * (size_t)n);
   L.range = take(sizeof(long) * 2 * (NBIN + 2));
   L.small = take(sizeof(int) * NSMALL * NBIN);
-  L.cell_of = take(4 * (size_t)n);
-  L.rec = take(8 * (size_t)ParkStride(method, BinMaxNM(method)) * (size_t)n);
+  const size_t recs = nrec ? (size_t)NBIN * nrec : (size_t)n;
+  L.cell_of = take(4 * recs);
+  L.rec = take(8 * (size_t)ParkStride(method, BinMaxNM(method)) * recs);
   size_t b = 0;
   const hipError_t e = hipcub::DeviceRadixSort::SortPairs(
       nullptr, b, (unsigned long long *)nullptr, (unsigned long long *)nullptr, (int *)nullptr,
@@ -89,8 +98,9 @@ hipError_t layout(int method, long n, Layout &L) {
 }
 
 hipError_t enqueue(int method, const PteArgs &a, const MixParamsDev &P,
-                   unsigned long long mod_mask, const Layout &L, BatchWs &ws, hipStream_t s) {
-  char *base = static_cast<char *>(ws.buf);
+                   unsigned long long mod_mask, int nrec, const Layout &L, void *buf,
+                   hipStream_t s) {
+  char *base = static_cast<char *>(buf);
   auto *keys = (unsigned long long *)(base + L.keys);
   auto *keys2 = (unsigned long long *)(base + L.keys2);
   int *ids = (int *)(base + L.ids), *sorted = (int *)(base + L.sorted);
@@ -104,81 +114,44 @@ hipError_t enqueue(int method, const PteArgs &a, const MixParamsDev &P,
   size_t tb = L.tmp_bytes;
   e = hipcub::DeviceRadixSort::SortPairs(base + L.tmp, tb, keys, keys2, ids, sorted, n, 0, 64, s);
   if (e != hipSuccess) return e;
-  batch_tables_kernel<<<1, 64, 0, s>>>(keys2, n, max_nm, range, small);
+  batch_tables_kernel<<<1, 64, 0, s>>>(keys2, n, max_nm, nrec, range, small);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((e = hipEventRecord(ws.ev[NBIN], s)) != hipSuccess) return e;
-  const int ncu = device_cu_count();
-  const int cpw = batch_cells_per_wave(n, ncu);
-  const int grid = (int)std::max<long>(1, std::min<long>((n + cpw - 1) / cpw, 8L * ncu));
-  // the longest tails first; a bin's tail follows it on the bin's stream
-  for (int nm = max_nm; nm >= 2; --nm) {
-    const int b = nm - 2;
-    hipStream_t q = ws.aux[b];
-    if ((e = hipStreamWaitEvent(q, ws.ev[NBIN], 0)) != hipSuccess) return e;
-    ParkArgs pk;
-    int *sm = small + NSMALL * b;
-    pk.after = BATCH_PARK_AFTER;
-    pk.stride = ParkStride(method, max_nm);
-    pk.rec = (double *)(base + L.rec);
-    pk.cell_of = (int *)(base + L.cell_of);
-    pk.run_base = sm;
-    pk.run_cap = sm + 1;
-    pk.run_count = sm + 2;
-    const int per_slot = 64 / TailGroup(method, nm);
-    pk.nwaves = (n + per_slot - 1) / per_slot;
-    pk.after2 = BATCH_AFTER2;
-    pk.l2_count = sm + 3;
-    pk.l2_next = sm + 4;
-    e = launch_pte_bin(method, nm, a, P, sorted, 0, sm + 5, 64, cpw, grid, q,
-                       range + 2 * (nm - 1), &pk);
-    if (e == hipSuccess) e = launch_pte_tail(method, nm, a, P, pk, q);
-    if (e == hipSuccess) e = hipEventRecord(ws.ev[b], q);
-    if (e != hipSuccess) return e;
-  }
-  for (int side = 0; side < 2; ++side)
-    if ((e = launch_pte_list(method, a, P, sorted, n, s,
-                             range + (side ? 2 * (NBIN + 1) : 0))) != hipSuccess)
-      return e;
-  for (int nm = max_nm; nm >= 2; --nm)
-    if ((e = hipStreamWaitEvent(s, ws.ev[nm - 2], 0)) != hipSuccess) return e;
-  return hipSuccess;
+  BatchArgs b;
+  b.small = small;
+  b.rec = (double *)(base + L.rec);
+  b.cell_of = (int *)(base + L.cell_of);
+  b.stride = ParkStride(method, max_nm);
+  b.after = BATCH_PARK_AFTER;
+  b.after2 = BATCH_AFTER2;
+  e = launch_pte_batch_bins(method, a, P, b, sorted, range, n,
+                            cells_per_wave(n, device_cu_count()), s);
+  for (int side = 0; side < 2 && e == hipSuccess; ++side)
+    e = launch_pte_list(method, a, P, sorted, n, s, range + (side ? 2 * (NBIN + 1) : 0));
+  return e;
 }
 
 } // namespace
 
-// Lanes of a wave that take cells: all 64 once the batch fills four waves per
-// CU with them, fewer below, where waves are plentiful and each pass of a
-// wave costs the sum of its lanes' material kinds.
-int batch_cells_per_wave(long ncell, int ncu) {
-  int c = 64;
-  while (c > 4 && ncell < 4L * ncu * c) c /= 2;
-  return c;
-}
-
 void BatchWs::release() {
-  if (done) (void)hipEventSynchronize(done);
+  if (done) {
+    (void)hipEventSynchronize(done);
+    (void)hipEventDestroy(done);
+  }
   if (buf) (void)hipFree(buf);
-  for (hipStream_t &q : aux)
-    if (q) (void)hipStreamDestroy(q);
-  for (hipEvent_t &v : ev)
-    if (v) (void)hipEventDestroy(v);
-  if (done) (void)hipEventDestroy(done);
   *this = BatchWs{};
 }
 
-namespace {
-bool make_streams(BatchWs &ws) {
-  if (ws.done) return true;
-  bool ok = true;
-  for (hipStream_t &q : ws.aux)
-    ok = ok && hipStreamCreateWithFlags(&q, hipStreamNonBlocking) == hipSuccess;
-  for (hipEvent_t &v : ws.ev)
-    ok = ok && hipEventCreateWithFlags(&v, hipEventDisableTiming) == hipSuccess;
-  ok = ok && hipEventCreateWithFlags(&ws.done, hipEventDisableTiming) == hipSuccess;
-  if (!ok) ws.release();
-  return ok;
+size_t batch_bytes(int method, long n, int nrec) {
+  Layout L;
+  return layout(method, n, nrec, L) == hipSuccess ? L.total : 0;
 }
-} // namespace
+
+hipError_t launch_batch(int method, const PteArgs &a, const MixParamsDev &P,
+                        unsigned long long mod_mask, int nrec, void *buf, hipStream_t s) {
+  Layout L;
+  const hipError_t e = layout(method, a.ncell, nrec, L);
+  return e != hipSuccess ? e : enqueue(method, a, P, mod_mask, nrec, L, buf, s);
+}
 
 hipError_t launch_pte_batch(sgm_ctx *ctx, int method, const PteArgs &a, const MixParamsDev &P,
                             hipStream_t s, bool &taken) {
@@ -190,7 +163,7 @@ hipError_t launch_pte_batch(sgm_ctx *ctx, int method, const PteArgs &a, const Mi
   }
   const long chunk = std::min<long>(a.ncell, BATCH_MAX_CELLS);
   Layout L;
-  if (layout(method, chunk, L) != hipSuccess) return hipSuccess;
+  if (layout(method, chunk, 0, L) != hipSuccess) return hipSuccess;
   std::lock_guard<std::mutex> g(ctx->batch_mu);
   // a workspace whose last call was on this stream or has finished, else a
   // new one, else the least recently used; its last call is waited for on the
@@ -207,7 +180,11 @@ hipError_t launch_pte_batch(sgm_ctx *ctx, int method, const PteArgs &a, const Mi
   }
   (void)hipGetLastError();  // a query of unfinished work
   if (!ws) ws = fresh ? fresh : oldest;
-  if (!make_streams(*ws)) return hipSuccess;
+  if (!ws->done && hipEventCreateWithFlags(&ws->done, hipEventDisableTiming) != hipSuccess) {
+    (void)hipGetLastError();
+    ws->done = nullptr;
+    return hipSuccess;
+  }
   if (ws->bytes < L.total) {
     if (hipEventSynchronize(ws->done) != hipSuccess) return hipSuccess;
     if (ws->buf) (void)hipFree(ws->buf);
@@ -238,7 +215,7 @@ hipError_t launch_pte_batch(sgm_ctx *ctx, int method, const PteArgs &a, const Mi
     if (b.niter) b.niter += c0;
     if (b.err) b.err += c0;
     if (b.resid) b.resid += c0;
-    e = enqueue(method, b, P, mods, L, *ws, s);
+    e = enqueue(method, b, P, mods, 0, L, ws->buf, s);
   }
   const hipError_t er = hipEventRecord(ws->done, s);
   return e != hipSuccess ? e : er;

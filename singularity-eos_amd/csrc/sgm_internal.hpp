@@ -30,14 +30,11 @@ struct VinetHost {
   Real *d_coef = nullptr;
 };
 
-// Work arrays, fork streams and events of one batched closure call
-// (sgm_batch.hip): one call at a time in stream order, `done` marking the
-// last one's end.
+// Work arrays of one batched closure call (sgm_batch.hip): one call at a time
+// in stream order, `done` marking the last one's end.
 struct BatchWs {
   void *buf = nullptr;
   size_t bytes = 0;
-  hipStream_t aux[5] = {};
-  hipEvent_t ev[6] = {};
   hipEvent_t done = nullptr;
   hipStream_t last = nullptr;
   unsigned long long used = 0;
@@ -102,7 +99,11 @@ inline unsigned long long ctx_mod_mask(const sgm_ctx *ctx) {
 // captured, or there is no memory for the work arrays).
 hipError_t launch_pte_batch(sgm_ctx *ctx, int method, const PteArgs &a, const MixParamsDev &P,
                             hipStream_t s, bool &taken);
-int batch_cells_per_wave(long ncell, int ncu);
+// the batch itself, its work arrays in buf (batch_bytes); nrec: straggler
+// records per material count, 0: one per cell
+size_t batch_bytes(int method, long n, int nrec);
+hipError_t launch_batch(int method, const PteArgs &a, const MixParamsDev &P,
+                        unsigned long long mod_mask, int nrec, void *buf, hipStream_t s);
 // MixParams as the kernels take them (NULL = the reference's defaults)
 MixParamsDev to_dev(const sgm_mix_params *p);
 // A batched plan over a CSR topology (sgm_plan_create) whose cells with fewer

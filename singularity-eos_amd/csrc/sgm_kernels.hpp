@@ -66,6 +66,18 @@ struct ParkArgs {
   int *l2_next = nullptr;           // second level (RhoT): next record item to take
 };
 
+// The tables of a batch (cells of every material count solved without a plan;
+// sgm_batch.hip): per material count 2..6 BATCH_SMALL ints {first record,
+// records, records claimed, level-2 cells, level-2 queue, cell counter}.
+constexpr int BATCH_SMALL = 6;
+struct BatchArgs {
+  int *small = nullptr;
+  double *rec = nullptr;
+  int *cell_of = nullptr;
+  int stride = 0;           // FP64 words per record, every material count alike
+  int after = 0, after2 = 0;  // as ParkArgs
+};
+
 // Closure formulations, by the method ids of the C ABI.
 enum PteMethod {
   PTE_RHOT = 0,
@@ -122,7 +134,10 @@ constexpr bool TailWide(int method, int nm) { return method == PTE_RHOT && nm >=
                                    int block, int cpw, int grid, const ParkArgs *park,         \
                                    hipStream_t s);                                             \
   hipError_t launch_pte_tail_##name(int nm, const PteArgs &a, const MixParamsDev &P,           \
-                                    const ParkArgs &park, hipStream_t s);
+                                    const ParkArgs &park, hipStream_t s);                      \
+  hipError_t launch_pte_batch_##name(const PteArgs &a, const MixParamsDev &P,                  \
+                                     const BatchArgs &b, const int *cells, const long *range,  \
+                                     long n, int chunk, hipStream_t s);
 SGM_PTE_LAUNCHERS(rhot)
 SGM_PTE_LAUNCHERS(pt)
 SGM_PTE_LAUNCHERS(fixedt)
@@ -202,6 +217,20 @@ inline hipError_t launch_pte_tail(int method, int nm, const PteArgs &a, const Mi
   case PTE_FIXED_T: return launch_pte_tail_fixedt(nm, a, P, park, s);
   case PTE_FIXED_P: return launch_pte_tail_fixedp(nm, a, P, park, s);
   case PTE_RHOU: return launch_pte_tail_rhou(nm, a, P, park, s);
+  default: return hipErrorInvalidValue;
+  }
+}
+// the bins and tails of a batch of n cells (range: per material count from 1,
+// {start, count} into `cells`, on the device)
+inline hipError_t launch_pte_batch_bins(int method, const PteArgs &a, const MixParamsDev &P,
+                                        const BatchArgs &b, const int *cells,
+                                        const long *range, long n, int chunk, hipStream_t s) {
+  switch (method) {
+  case PTE_RHOT: return launch_pte_batch_rhot(a, P, b, cells, range, n, chunk, s);
+  case PTE_PT: return launch_pte_batch_pt(a, P, b, cells, range, n, chunk, s);
+  case PTE_FIXED_T: return launch_pte_batch_fixedt(a, P, b, cells, range, n, chunk, s);
+  case PTE_FIXED_P: return launch_pte_batch_fixedp(a, P, b, cells, range, n, chunk, s);
+  case PTE_RHOU: return launch_pte_batch_rhou(a, P, b, cells, range, n, chunk, s);
   default: return hipErrorInvalidValue;
   }
 }

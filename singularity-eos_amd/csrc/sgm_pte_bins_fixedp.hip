@@ -10,4 +10,9 @@ hipError_t launch_pte_tail_fixedp(int nm, const PteArgs &a, const MixParamsDev &
                               const ParkArgs &park, hipStream_t s) {
   return kern::tail_launch<3>(nm, a, P, park, s);
 }
+hipError_t launch_pte_batch_fixedp(const PteArgs &a, const MixParamsDev &P, const BatchArgs &b,
+                               const int *cells, const long *range, long n, int chunk,
+                               hipStream_t s) {
+  return kern::batch_launch<3>(a, P, b, cells, range, n, chunk, s);
+}
 } // namespace sgm

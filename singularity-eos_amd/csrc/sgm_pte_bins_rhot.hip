@@ -10,4 +10,9 @@ hipError_t launch_pte_tail_rhot(int nm, const PteArgs &a, const MixParamsDev &P,
                               const ParkArgs &park, hipStream_t s) {
   return kern::tail_launch<0>(nm, a, P, park, s);
 }
+hipError_t launch_pte_batch_rhot(const PteArgs &a, const MixParamsDev &P, const BatchArgs &b,
+                               const int *cells, const long *range, long n, int chunk,
+                               hipStream_t s) {
+  return kern::batch_launch<0>(a, P, b, cells, range, n, chunk, s);
+}
 } // namespace sgm

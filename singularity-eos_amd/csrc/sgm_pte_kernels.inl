@@ -236,18 +236,10 @@ constexpr int REFILL_BATCH = 1;
 #define SGM_BIN_WAVES_PER_EU 2
 #endif
 template <int NM, int METHOD>
-__global__ void __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(SGM_BIN_WAVES_PER_EU,
-                                   SGM_BIN_WAVES_PER_EU))) pte_bin_kernel(PteArgs a, MixParamsDev P,
-                                                      const int *__restrict__ cells,
-                                                      long ncells, int *counter, int chunk,
-                                                      const long *range, ParkArgs pk) {
-  extern __shared__ EosDev lds[];
-  stage_registry(lds, a.d_eos, a.nreg);
-  if (range) {  // bin bounds computed on the device: {start, count} into cells
-    cells += range[0];
-    ncells = range[1];
-  }
+__device__ __forceinline__ void bin_body(const EosDev *lds, const PteArgs &a,
+                                         const MixParamsDev &P, const int *__restrict__ cells,
+                                         long ncells, int *counter, int chunk,
+                                         const ParkArgs &pk) {
   const int lane = threadIdx.x & 63;
   const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   // a claim covers every lane that takes cells: fewer than 64 cells per claim
@@ -329,6 +321,22 @@ __attribute__((amdgpu_waves_per_eu(SGM_BIN_WAVES_PER_EU,
       park_ok = false;
     }
   }
+}
+
+template <int NM, int METHOD>
+__global__ void __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(SGM_BIN_WAVES_PER_EU,
+                                   SGM_BIN_WAVES_PER_EU))) pte_bin_kernel(PteArgs a, MixParamsDev P,
+                                                      const int *__restrict__ cells,
+                                                      long ncells, int *counter, int chunk,
+                                                      const long *range, ParkArgs pk) {
+  extern __shared__ EosDev lds[];
+  stage_registry(lds, a.d_eos, a.nreg);
+  if (range) {  // bin bounds computed on the device: {start, count} into cells
+    cells += range[0];
+    ncells = range[1];
+  }
+  bin_body<NM, METHOD>(lds, a, P, cells, ncells, counter, chunk, pk);
 }
 
 // Resumes the parked cells of one bin in two levels. Level 1 (LEVEL 1): a
@@ -416,15 +424,11 @@ __device__ __forceinline__ void tail_wide(const PteArgs &a, const MixParamsDev &
   }
 }
 
-template <int NM, int METHOD, int WPE, int LEVEL>
-__global__ void __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(WPE, WPE))) pte_tail_kernel(PteArgs a, MixParamsDev P,
-                                                                ParkArgs pk, int resident,
-                                                                int wide_max) {
+template <int NM, int METHOD, int LEVEL>
+__device__ __forceinline__ void tail_body(const PteArgs &a, const MixParamsDev &P,
+                                          const ParkArgs &pk, int resident, int wide_max) {
   constexpr int G = TailGroup(METHOD, NM);
   constexpr int per_slot = 64 / G;  // records per wave slot
-  extern __shared__ EosDev lds[];
-  stage_registry(lds, a.d_eos, a.nreg);
   const int lane = (int)threadIdx.x;
   const bool two_levels = G > 1 && pk.after2 > 0 && pk.l2_count && P.line_search_max_iter <= G;
   if constexpr (LEVEL == 3) {
@@ -520,6 +524,102 @@ __attribute__((amdgpu_waves_per_eu(WPE, WPE))) pte_tail_kernel(PteArgs a, MixPar
       }
     }
   }
+}
+
+template <int NM, int METHOD, int WPE, int LEVEL>
+__global__ void __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(WPE, WPE))) pte_tail_kernel(PteArgs a, MixParamsDev P,
+                                                                ParkArgs pk, int resident,
+                                                                int wide_max) {
+  extern __shared__ EosDev lds[];
+  stage_registry(lds, a.d_eos, a.nreg);
+  tail_body<NM, METHOD, LEVEL>(a, P, pk, resident, wide_max);
+}
+
+// All bins of a batch in one launch (blockIdx.y: the material count, largest
+// first), its bounds and records read from the batch's tables. Bins of their
+// own kernels would need a stream each to run side by side, and the process
+// has four hardware queues: the fifth bin, and any other batch in flight,
+// would wait behind a queue's tails. The bins' kernels need the same
+// registers one by one as together.
+template <int NM>
+__device__ __forceinline__ ParkArgs batch_park(const BatchArgs &b) {
+  ParkArgs pk;
+  int *sm = b.small + BATCH_SMALL * (NM - 2);
+  pk.after = b.after;
+  pk.stride = b.stride;
+  pk.rec = b.rec;
+  pk.cell_of = b.cell_of;
+  pk.run_base = sm;
+  pk.run_cap = sm + 1;
+  pk.run_count = sm + 2;
+  pk.nwaves = 0;  // one run: its claimed records
+  pk.after2 = b.after2;
+  pk.l2_count = sm + 3;
+  pk.l2_next = sm + 4;
+  return pk;
+}
+template <int METHOD>
+__global__ void __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(SGM_BIN_WAVES_PER_EU, SGM_BIN_WAVES_PER_EU)))
+pte_batch_bins_kernel(PteArgs a, MixParamsDev P, BatchArgs b, const int *__restrict__ cells,
+                      const long *__restrict__ range, int chunk) {
+  extern __shared__ EosDev lds[];
+  const int nm = BinMaxNM(METHOD) - (int)blockIdx.y;
+  const long *r = range + 2 * (nm - 1);
+  if ((long)blockIdx.x * chunk >= r[1]) return;  // more waves than the bin's cells fill
+  stage_registry(lds, a.d_eos, a.nreg);
+#define SGM_ONE(K)                                                                             \
+  case K:                                                                                      \
+    if constexpr (K <= BinMaxNM(METHOD))                                                       \
+      bin_body<K, METHOD>(lds, a, P, cells + r[0], r[1], b.small + BATCH_SMALL * (K - 2) + 5,  \
+                          chunk, batch_park<K>(b));                                            \
+    break;
+  switch (nm) { SGM_ONE(2) SGM_ONE(3) SGM_ONE(4) SGM_ONE(5) SGM_ONE(6) }
+#undef SGM_ONE
+}
+// level 1 (LEVEL 1), then level 2 in the form each bin's population asks for
+template <int METHOD, int LEVEL>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, LEVEL == 1 ? 2 : 1)))
+pte_batch_tails_kernel(PteArgs a, MixParamsDev P, BatchArgs b, int resident, int wide_max) {
+  extern __shared__ EosDev lds[];
+  const int nm = BinMaxNM(METHOD) - (int)blockIdx.y;
+  const int *sm = b.small + BATCH_SMALL * (nm - 2);
+  if (sm[2] == 0 || (LEVEL == 2 && sm[3] == 0)) return;  // nothing parked
+  stage_registry(lds, a.d_eos, a.nreg);
+#define SGM_ONE(K)                                                                             \
+  case K:                                                                                      \
+    if constexpr (K <= BinMaxNM(METHOD)) {                                                     \
+      const ParkArgs pk = batch_park<K>(b);                                                    \
+      if constexpr (LEVEL == 2 && TailWide(METHOD, K)) {                                       \
+        if ((int)blockIdx.x < wide_max / 4) tail_body<K, METHOD, 3>(a, P, pk, resident, wide_max); \
+      }                                                                                        \
+      if constexpr (LEVEL == 1 || TailGroup(METHOD, K) > 1)                                    \
+        tail_body<K, METHOD, LEVEL>(a, P, pk, resident, wide_max);                             \
+    }                                                                                          \
+    break;
+  switch (nm) { SGM_ONE(2) SGM_ONE(3) SGM_ONE(4) SGM_ONE(5) SGM_ONE(6) }
+#undef SGM_ONE
+}
+
+template <int METHOD>
+hipError_t batch_launch(const PteArgs &a, const MixParamsDev &P, const BatchArgs &b,
+                        const int *cells, const long *range, long n, int chunk, hipStream_t s) {
+  const size_t lds = (size_t)a.nreg * sizeof(EosDev);
+  const int ncu = device_cu_count();
+  const int nbin = BinMaxNM(METHOD) - 1;
+  const long waves = (n + chunk - 1) / chunk;
+  const int g = (int)(waves < 8L * ncu ? waves : 8L * ncu);
+  pte_batch_bins_kernel<METHOD><<<dim3(g, nbin), 64, lds, s>>>(a, P, b, cells, range, chunk);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || b.after <= 0) return e;
+  const int gt = (int)(n < 4L * ncu ? n : 4L * ncu);
+  pte_batch_tails_kernel<METHOD, 1><<<dim3(gt, nbin), 64, lds, s>>>(a, P, b, 4 * ncu, 4 * ncu);
+  e = hipGetLastError();
+  if (e != hipSuccess || TailGroup(METHOD, 2) == 1 || P.line_search_max_iter > TailGroup(METHOD, 2))
+    return e;
+  pte_batch_tails_kernel<METHOD, 2><<<dim3(gt, nbin), 64, lds, s>>>(a, P, b, 4 * ncu, 4 * ncu);
+  return hipGetLastError();
 }
 
 template <int METHOD>

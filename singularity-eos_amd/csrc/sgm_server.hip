@@ -5,18 +5,15 @@
 // on the lane's stream and the scheduler thread only polls the lane's event:
 //   H2D   request table, each closure request's raw offsets and per-entry /
 //         per-cell inputs into one merged CSR, each vector request's inputs
-//   ker   offsets rebase (merged CSR), sort keys, radix sort, bin bounds,
-//         counter reset, one persistent bin kernel per material count 2..6
-//         with straggler parking and the bin's tail kernels behind it, and
-//         the list kernel for the rest (bin bounds read on the device);
-//         one vector kernel per vector request
+//   ker   offsets rebase (merged CSR), then the cells as one batch
+//         (sgm_batch.hip: all material counts side by side in one kernel per
+//         stage, so a group needs no stream but its lane's); one vector
+//         kernel per vector request
 //   D2H   results straight into the clients' arrays
 // Admission is first-come first-served: the queue head waits until its
 // working set fits in a free stretch of the arena; a request larger than the
 // whole arena is refused at submit.
 #include "sgm_internal.hpp"
-
-#include <hipcub/hipcub.hpp>
 
 #include <algorithm>
 #include <atomic>
@@ -33,8 +30,6 @@ using namespace sgm;
 namespace {
 
 constexpr size_t ALIGN = 256;
-// Newton iterations before a bin kernel parks a cell (as plans do)
-constexpr int SERVER_PARK_AFTER = 20;
 inline size_t align_up(size_t x) { return (x + ALIGN - 1) & ~(ALIGN - 1); }
 
 // device-side description of one closure request inside a group
@@ -65,52 +60,6 @@ __global__ void rebase_kernel(const ReqDev *__restrict__ reqs, int nreq,
   // offsets outside the request's own entry range mark the cell invalid
   // (the solver then flags it and touches no other request's entries)
   off[g] = (ri >= r0 && ri <= rn) ? (int)(r.nnz_base + (ri - r0)) : -1;
-}
-
-// bin bounds of sorted keys (nmat << 56 | signature): range[2k..] = {start,
-// count} for k = 0: nmat < 2, 1..5: nmat = k+1, 6: nmat > 6 (incl. invalid)
-__global__ void ranges_kernel(const unsigned long long *__restrict__ keys, long n,
-                              long *__restrict__ range) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  long pos[7];
-  for (int nm = 2; nm <= 8; ++nm) {
-    const unsigned long long k = (unsigned long long)nm << 56;
-    long lo = 0, hi = n;  // first index with keys[i] >= k
-    while (lo < hi) {
-      const long mid = (lo + hi) >> 1;
-      if (keys[mid] < k)
-        lo = mid + 1;
-      else
-        hi = mid;
-    }
-    pos[nm - 2] = lo;
-  }
-  range[0] = 0;
-  range[1] = pos[0];
-  for (int b = 1; b <= 5; ++b) {
-    range[2 * b] = pos[b - 1];
-    range[2 * b + 1] = pos[b] - pos[b - 1];
-  }
-  range[12] = pos[5];
-  range[13] = n - pos[5];
-}
-
-// The straggler tables of a launch group. The group's bins are not split by
-// material signature, so each bin is one run: every position maps to run 0
-// (run_of), the tail's wave slots walk the bin's records in park order
-// (wave_run 0, wave_first = slot x per_wave), and per bin `small` holds
-// {run_base 0, run_cap R, run_count 0, level-2 count 0, level-2 queue 0}.
-__global__ void park_tables_kernel(int *__restrict__ run_of, long ncell,
-                                   int *__restrict__ wave_run, int *__restrict__ wave_first,
-                                   int nw, int per_wave, int *__restrict__ small, int nsmall,
-                                   int R) {
-  const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g < ncell) run_of[g] = 0;
-  if (g < nw) {
-    wave_run[g] = 0;
-    wave_first[g] = (int)g * per_wave;
-  }
-  if (g < nsmall) small[g] = (g % 5 == 1) ? R : 0;
 }
 
 struct Arena {
@@ -170,13 +119,8 @@ struct Rec {
 struct Layout {
   long ncell = 0, nnz = 0, nraw = 0;
   int npte = 0;
-  size_t reqs, raw, off, mat, rho, vfrac, sie, temp, press, vt, st, conv, keys, keys2, ids,
-      sorted, range, counters, sort_tmp, sort_tmp_bytes;
-  // straggler parking of the batched bins (2..6 materials): R records per bin
-  long park_R = 0;
-  int park_nw = 0, park_per_wave = 0;
-  size_t run_of = 0, wave_run = 0, wave_first = 0, park_small = 0;
-  size_t rec[7] = {}, cell_of[7] = {};
+  size_t reqs, raw, off, mat, rho, vfrac, sie, temp, press, vt, st, conv, batch = 0;
+  int nrec = 0;  // straggler records per material count
   std::vector<size_t> vec_in, vec_out;  // per vector request: rho, sie | P, T
   size_t total = 0;
 };
@@ -219,14 +163,6 @@ struct sgm_server {
 
 namespace {
 
-size_t sort_tmp_bytes(long n) {
-  size_t b = 0;
-  hipcub::DeviceRadixSort::SortPairs(nullptr, b, (unsigned long long *)nullptr,
-                                     (unsigned long long *)nullptr, (int *)nullptr,
-                                     (int *)nullptr, (int)std::max<long>(n, 1), 0, 64);
-  return b + 16;
-}
-
 Layout make_layout(const sgm_server *sv, const std::vector<uint64_t> &ids) {
   Layout L;
   size_t o = 0;
@@ -260,30 +196,12 @@ Layout make_layout(const sgm_server *sv, const std::vector<uint64_t> &ids) {
     L.vt = take(8 * L.ncell);
     L.st = take(8 * L.ncell);
     L.conv = take(4 * L.ncell);
-    L.keys = take(8 * L.ncell);
-    L.keys2 = take(8 * L.ncell);
-    L.ids = take(4 * L.ncell);
-    L.sorted = take(4 * L.ncell);
-    L.range = take(sizeof(long) * 14);
-    L.counters = take(sizeof(int) * 8);
-    L.sort_tmp_bytes = sort_tmp_bytes(L.ncell);
-    L.sort_tmp = take(L.sort_tmp_bytes);
     if (!sv->cfg.plain) {
-      // records for a sixteenth of the group's cells per bin (at least 1024):
-      // a cell still iterating after SERVER_PARK_AFTER Newton iterations moves
-      // to the bin's tail kernels while records last, and keeps its lane past
-      // that
-      L.park_R = std::min<long>(L.ncell, std::max<long>(1024, L.ncell / 16));
-      L.park_per_wave = 64 / TailGroup(sv->cfg.method, 2);
-      L.park_nw = (int)((L.park_R + L.park_per_wave - 1) / L.park_per_wave);
-      L.run_of = take(4 * L.ncell);
-      L.wave_run = take(4 * (size_t)L.park_nw);
-      L.wave_first = take(4 * (size_t)L.park_nw);
-      L.park_small = take(4 * 5 * 5);
-      for (int nm = 2; nm <= 6; ++nm) {
-        L.rec[nm] = take(8 * (size_t)ParkStride(sv->cfg.method, nm) * L.park_R);
-        L.cell_of[nm] = take(4 * (size_t)L.park_R);
-      }
+      // records for a twenty-second of the group's cells per material count
+      // (at least 776): a cell still iterating after the batch's threshold
+      // moves to its tail while records last, and keeps its lane past that
+      L.nrec = (int)std::max<long>(776, L.ncell / 22);
+      L.batch = take(batch_bytes(sv->cfg.method, L.ncell, L.nrec));
     }
   }
   for (uint64_t t : ids) {
@@ -362,54 +280,7 @@ int launch_group(sgm_server *sv, Lane &ln, const Layout &L) {
     if (sv->cfg.plain) {
       ok(launch_pte_plain(sv->cfg.method, a, sv->P, s));
     } else {
-      auto *keys = (unsigned long long *)D(L.keys), *keys2 = (unsigned long long *)D(L.keys2);
-      int *ids = (int *)D(L.ids), *sorted = (int *)D(L.sorted);
-      long *range = (long *)D(L.range);
-      int *counters = (int *)D(L.counters);
-      ok(launch_plan_keys(off, a.mat_ids, L.ncell, L.nnz, keys, ids, s, nullptr, 0,
-                          ctx_mod_mask(ctx)));
-      size_t tb = L.sort_tmp_bytes;
-      ok(hipcub::DeviceRadixSort::SortPairs(D(L.sort_tmp), tb, keys, keys2, ids, sorted,
-                                            (int)L.ncell, 0, 64, s));
-      ranges_kernel<<<1, 64, 0, s>>>(keys2, L.ncell, range);
-      ok(hipGetLastError());
-      ok(launch_zero_ints(counters, 8, s));
-      const int grid = std::max(1, sv->ncu * 2);  // 8 waves per CU of 256-thread blocks
-      int *small = (int *)D(L.park_small);
-      const long nt = std::max<long>(std::max<long>(L.ncell, L.park_nw), 25);
-      park_tables_kernel<<<(int)((nt + 255) / 256), 256, 0, s>>>(
-          (int *)D(L.run_of), L.ncell, (int *)D(L.wave_run), (int *)D(L.wave_first), L.park_nw,
-          L.park_per_wave, small, 25, (int)L.park_R);
-      ok(hipGetLastError());
-      // each bin's persistent kernel parks its stragglers, then the bin's
-      // tail kernels finish them (as a plan does, on the lane's stream), so
-      // a few wandering cells no longer hold the bin kernel's whole grid
-      for (int nm = 2; nm <= 6; ++nm) {
-        const long *r = range + 2 * (nm - 1);
-        ParkArgs pk;
-        int *sm = small + 5 * (nm - 2);
-        pk.after = SERVER_PARK_AFTER;
-        pk.stride = ParkStride(sv->cfg.method, nm);
-        pk.rec = (double *)D(L.rec[nm]);
-        pk.cell_of = (int *)D(L.cell_of[nm]);
-        pk.run_of = (const int *)D(L.run_of);
-        pk.run_base = sm;
-        pk.run_cap = sm + 1;
-        pk.run_count = sm + 2;
-        pk.wave_run = (const int *)D(L.wave_run);
-        pk.wave_first = (const int *)D(L.wave_first);
-        pk.nwaves = L.park_nw;
-        pk.after2 = 4;
-        pk.l2_count = sm + 3;
-        pk.l2_next = sm + 4;
-        ok(launch_pte_bin(sv->cfg.method, nm, a, sv->P, sorted, 0, counters + nm, 256, 64, grid,
-                          s, r, &pk));
-        ok(launch_pte_tail(sv->cfg.method, nm, a, sv->P, pk, s));
-      }
-      for (int side = 0; side < 2; ++side) {
-        const long *r = range + (side ? 12 : 0);
-        ok(launch_pte_list(sv->cfg.method, a, sv->P, sorted, L.ncell, s, r));
-      }
+      ok(launch_batch(sv->cfg.method, a, sv->P, ctx_mod_mask(ctx), L.nrec, D(L.batch), s));
     }
     if (e != hipSuccess) return SGM_E_HIP;
     cb = 0;
