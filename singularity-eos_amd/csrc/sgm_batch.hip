@@ -15,6 +15,15 @@
 #include <algorithm>
 
 namespace sgm {
+// Lanes of a wave that take cells: all 64 once the batch fills four waves per
+// CU with them, fewer below, where waves are plentiful and each pass of a
+// wave costs the sum of its lanes' material kinds.
+int batch_cells_per_wave(long ncell, int ncu) {
+  int c = 64;
+  while (c > 4 && ncell < 4L * ncu * c) c /= 2;
+  return c;
+}
+
 namespace {
 
 constexpr int NBIN = 5, NSMALL = BATCH_SMALL;  // bins: material counts 2..6
@@ -56,15 +65,6 @@ __global__ void batch_tables_kernel(const unsigned long long *__restrict__ keys,
     range[2 * NBIN + 2] = pos[NBIN];
     range[2 * NBIN + 3] = n - pos[NBIN];
   }
-}
-
-// Lanes of a wave that take cells: all 64 once the batch fills four waves per
-// CU with them, fewer below, where waves are plentiful and each pass of a
-// wave costs the sum of its lanes' material kinds.
-int cells_per_wave(long ncell, int ncu) {
-  int c = 64;
-  while (c > 4 && ncell < 4L * ncu * c) c /= 2;
-  return c;
 }
 
 struct Layout {
@@ -124,7 +124,7 @@ hipError_t enqueue(int method, const PteArgs &a, const MixParamsDev &P,
   b.after = BATCH_PARK_AFTER;
   b.after2 = BATCH_AFTER2;
   e = launch_pte_batch_bins(method, a, P, b, sorted, range, n,
-                            cells_per_wave(n, device_cu_count()), s);
+                            batch_cells_per_wave(n, device_cu_count()), s);
   for (int side = 0; side < 2 && e == hipSuccess; ++side)
     e = launch_pte_list(method, a, P, sorted, n, s, range + (side ? 2 * (NBIN + 1) : 0));
   return e;

@@ -50,7 +50,13 @@ struct sgm_plan {
   int *d_run_of = nullptr, *d_run_base = nullptr, *d_run_cap = nullptr;
   int *d_run_count = nullptr, *d_wave_run = nullptr, *d_wave_first = nullptr;
   int nruns = 0;
-  int *d_l2_counts = nullptr;    // per bin: cells saved for the tail's second level, its queue
+  // straggler records of all bins (one stride), and the tables of a launch
+  // whose bins share one kernel (BatchArgs): per material count its first
+  // record, records, and the counters of the last execution
+  double *d_rec = nullptr;
+  int *d_cell_of = nullptr, *d_small = nullptr;
+  long *d_range = nullptr;
+  bool own_shape = false;  // a launch shape was set: the bins keep their own kernels
   int *d_flag = nullptr;         // plan_match's result
   int park_after = 20;           // Newton iterations before a cell is parked; 0 = never
   std::vector<Bin> bins;
@@ -152,16 +158,38 @@ hipError_t alloc_park(sgm_plan *p, const std::vector<unsigned long long> &keys) 
   if (e == hipSuccess) e = up(&p->d_run_count, run_cap);  // contents reset per execution
   if (e == hipSuccess) e = up(&p->d_wave_run, wave_run);
   if (e == hipSuccess) e = up(&p->d_wave_first, wave_first);
+  long total = 0;
+  for (long n : nrec) total += n;
+  const int stride = ParkStride(p->method, BinMaxNM(p->method));
+  if (e == hipSuccess && total > 0)
+    e = hipMalloc(&p->d_rec, sizeof(double) * stride * (size_t)total);
+  if (e == hipSuccess && total > 0) e = hipMalloc(&p->d_cell_of, sizeof(int) * total);
+  std::vector<int> small(5 * BATCH_SMALL, 0);
+  std::vector<long> range(14, 0);
+  long first = 0;
+  for (size_t bi = 0; bi < p->bins.size(); ++bi) {
+    const Bin &b = p->bins[bi];
+    if (b.nm < 2 || b.nm > 6) continue;
+    small[BATCH_SMALL * (b.nm - 2)] = (int)first;
+    small[BATCH_SMALL * (b.nm - 2) + 1] = (int)nrec[bi];
+    range[2 * (b.nm - 1)] = b.start;
+    range[2 * (b.nm - 1) + 1] = b.n;
+    first += nrec[bi];
+  }
+  if (e == hipSuccess) e = up(&p->d_small, small);
+  if (e == hipSuccess) e = hipMalloc(&p->d_range, sizeof(long) * range.size());
   if (e == hipSuccess)
-    e = hipMalloc(&p->d_l2_counts, sizeof(int) * 2 * std::max<size_t>(1, p->bins.size()));
+    e = hipMemcpy(p->d_range, range.data(), sizeof(long) * range.size(), hipMemcpyHostToDevice);
+  first = 0;
   for (size_t bi = 0; bi < p->bins.size() && e == hipSuccess; ++bi) {
     Bin &b = p->bins[bi];
     if (b.nm < 2 || b.nm > 6 || nrec[bi] == 0) continue;
     ParkArgs &k = b.park;
-    k.stride = ParkStride(p->method, b.nm);
-    e = hipMalloc(&k.rec, sizeof(double) * k.stride * (size_t)nrec[bi]);
-    if (e == hipSuccess) e = hipMalloc(&k.cell_of, sizeof(int) * nrec[bi]);
-    k.l2_count = p->d_l2_counts + 2 * bi;
+    k.stride = stride;
+    k.rec = p->d_rec + first * stride;
+    k.cell_of = p->d_cell_of + first;
+    first += nrec[bi];
+    k.l2_count = p->d_small + BATCH_SMALL * (b.nm - 2) + 3;
     k.l2_next = k.l2_count + 1;
     k.after2 = 4;
     k.run_of = p->d_run_of + b.start;
@@ -179,28 +207,34 @@ hipError_t alloc_park(sgm_plan *p, const std::vector<unsigned long long> &keys) 
 // later failed alloc_park or sgm_plan_destroy never frees them twice
 void free_park(sgm_plan *p) {
   for (Bin &b : p->bins) {
-    for (void *q : {(void *)b.park.rec, (void *)b.park.cell_of})
-      if (q) (void)hipFree(q);
     b.park.rec = nullptr;
     b.park.cell_of = nullptr;
   }
+  for (void *q : {(void *)p->d_rec, (void *)p->d_range})
+    if (q) (void)hipFree(q);
+  p->d_rec = nullptr;
+  p->d_range = nullptr;
   for (int **q : {&p->d_run_of, &p->d_run_base, &p->d_run_cap, &p->d_run_count, &p->d_wave_run,
-                  &p->d_wave_first, &p->d_l2_counts}) {
+                  &p->d_wave_first, &p->d_cell_of, &p->d_small}) {
     if (*q) (void)hipFree(*q);
     *q = nullptr;
   }
 }
 
-// Resets the bin counters and the straggler claim counters (fill kernels, so
-// the resets can be captured).
+// Zeroes the bin counters, the straggler claim counters and the batch tables'
+// counters (with parking off too: sgm_plan_tail_counts then reports zeros). A
+// fill kernel, so the reset can be captured.
+__global__ void reset_kernel(int *counters, int nbins, int *run_count, int nruns, int *small) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < nbins) counters[i] = 0;
+  if (run_count && i < nruns) run_count[i] = 0;
+  if (small && i < 5 * BATCH_SMALL && i % BATCH_SMALL >= 2) small[i] = 0;
+}
 hipError_t reset_counters(sgm_plan *p, hipStream_t s) {
-  hipError_t e = launch_zero_ints(p->d_counters, (int)p->bins.size(), s);
-  if (e == hipSuccess && p->park_after > 0 && p->nruns > 0)
-    e = launch_zero_ints(p->d_run_count, p->nruns, s);
-  // cleared with parking off too: sgm_plan_tail_counts then reports zeros
-  if (e == hipSuccess && p->d_l2_counts)
-    e = launch_zero_ints(p->d_l2_counts, 2 * (int)p->bins.size(), s);
-  return e;
+  const int n = std::max(std::max((int)p->bins.size(), p->nruns), 5 * BATCH_SMALL);
+  reset_kernel<<<(n + 255) / 256, 256, 0, s>>>(p->d_counters, (int)p->bins.size(),
+                                                p->d_run_count, p->nruns, p->d_small);
+  return hipGetLastError();
 }
 
 // A list bin: the plain solver over its cells, one lane per cell, or one
@@ -245,6 +279,14 @@ std::vector<size_t> bin_order(const sgm_plan *p) {
   return order;
 }
 
+// Plans of up to this many cells launch their bins together (one kernel for
+// all bins, one per tail level: launch_pte_batch_bins): their bins do not
+// fill the GPU one by one. Larger ones overlap each bin's tail with the next
+// bins' kernels. Together against forked: 2^17 cells
+// of get_sg_eos 63 -> 55 ms, plans of 2,517 cells 10.2 -> 4.7 ms, 142,921 14.6 -> 13.1,
+// 2^18 15.5 -> 13.7.
+constexpr long PLAN_MERGED_CELLS = 1L << 18;
+
 // Records the counter reset and every bin on stream s: the persistent bin
 // kernels one after another on s; with fork streams (graph capture, or a
 // direct launch that may overlap) each bin's tail kernel forks off to a
@@ -254,6 +296,21 @@ hipError_t launch_bins(sgm_plan *p, const PteArgs &a, const MixParamsDev &P, hip
                        bool fork) {
   hipError_t e = reset_counters(p, s);
   if (e != hipSuccess) return e;
+  if (p->ncell <= PLAN_MERGED_CELLS && !p->own_shape && p->d_rec) {
+    BatchArgs b;
+    b.small = p->d_small;
+    b.rec = p->d_rec;
+    b.cell_of = p->d_cell_of;
+    b.stride = ParkStride(p->method, BinMaxNM(p->method));
+    b.after = p->park_after;
+    b.after2 = 4;
+    e = launch_pte_batch_bins(p->method, a, P, b, p->d_sorted, p->d_range, p->ncell,
+                              batch_cells_per_wave(p->ncell, device_cu_count()), s);
+    for (const Bin &x : p->bins)
+      if (e == hipSuccess && (x.nm < 2 || x.nm > 6))
+        e = launch_list_bin(p, x, a, P, p->d_sorted + x.start, s);
+    return e;
+  }
   const std::vector<size_t> order = bin_order(p);
   const size_t nb = p->bins.size();
   fork = fork && p->aux.size() >= nb && p->ev.size() >= 2 * nb;
@@ -492,15 +549,16 @@ int sgm_plan_describe(const sgm_plan *p, long *out, int max_bins) {
 int sgm_plan_tail_counts(const sgm_plan *p, int *out, int max_bins, sgm_stream_t stream) {
   if (!p || !out || max_bins < 0) return SGM_E_ARG;
   const int nb = (int)p->bins.size();
-  std::vector<int> c(2 * (size_t)std::max(1, nb), 0);
-  if (p->d_l2_counts) {
+  std::vector<int> c(5 * BATCH_SMALL, 0);
+  if (p->d_small) {
     hipStream_t s = (hipStream_t)stream;
-    if (hipMemcpyAsync(c.data(), p->d_l2_counts, sizeof(int) * c.size(), hipMemcpyDeviceToHost,
-                       s) != hipSuccess ||
+    if (hipMemcpyAsync(c.data(), p->d_small, sizeof(int) * c.size(), hipMemcpyDeviceToHost, s) !=
+            hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
       return SGM_E_HIP;
   }
-  for (int i = 0; i < nb && i < max_bins; ++i) out[i] = p->bins[i].park.rec ? c[2 * i] : 0;
+  for (int i = 0; i < nb && i < max_bins; ++i)
+    out[i] = p->bins[i].park.rec ? c[BATCH_SMALL * (p->bins[i].nm - 2) + 3] : 0;
   return nb;
 }
 
@@ -634,6 +692,7 @@ int sgm_plan_autotune(sgm_plan *p, const double *rho, const double *vfrac, const
           }
         }
     b = bestb;
+    p->own_shape = true;
   }
   hipEventDestroy(e0);
   hipEventDestroy(e1);
@@ -760,6 +819,7 @@ int sgm_plan_set_shape(sgm_plan *p, int bin, int block, int cells_per_wave, int 
   b.block = block;
   b.cpw = cells_per_wave;
   b.grid = grid;
+  p->own_shape = true;
   p->have_key = false;
   return SGM_OK;
 }
