@@ -2011,6 +2011,203 @@ SGM_HD void skip_to_last_pass(DriverState &d) {
   if (d.niter < d.max_iter - 1) d.niter = d.max_iter - 1;
 }
 
+// PTESolverPT for one cell on a team of NM waves, wave m holding material m: a
+// pass inverts each material's (P, T)
+// two times for the Jacobian and once per trial, 11 to 15 us each for a
+// Gruneisen, Vinet or table material on one wave, and the inversions of one
+// material start from its own last density only. So the materials' chains
+// run side by side on the CU's SIMDs, and every wave forms the sums from the
+// terms the team exchanges through LDS, in material order: the values and
+// the control flow are those of PtePT on every wave alike. Has the interface
+// pte_step drives.
+template <int NM>
+struct TeamPT {
+  using Ev = sgm::Ev<false>;
+  using Base = PtePT<NM, false>;
+  struct Shared {
+    Real x[2][4][NM];
+  };
+  Shared *sh;
+  int turn;  // the exchange buffer in use: two alternate, one barrier each
+  int m;     // this wave's material
+  unsigned char eidx[NM];
+  Lam lam;
+  Real rho, vfrac, sie, u, rhobar;
+  Real res[2], dx[2], jac[4];
+  Real vfrac_total, uscale, utotal_scale, Tnorm, Pequil, Tequil, Ptemp, Ttemp;
+  int err;
+  MixParamsDev P;
+
+  __device__ __forceinline__ const EosDev &E(int k) const { return registry_entry(eidx[k]); }
+  // turn0: the buffer after the team's last exchange
+  __device__ __forceinline__ void Take(const Base &b, int wave, Shared *shared, int turn0) {
+    sh = shared;
+    turn = turn0;
+    m = wave;
+#pragma unroll
+    for (int k = 0; k < NM; ++k) eidx[k] = b.eidx[k];
+    lam = b.lam[0];
+#pragma unroll
+    for (int k = 1; k < NM; ++k) {
+      lam.lRho = sel(m == k, b.lam[k].lRho, lam.lRho);
+      lam.lT = sel(m == k, b.lam[k].lT, lam.lT);
+    }
+    rho = pick<NM>(b.rho, m);
+    vfrac = pick<NM>(b.vfrac, m);
+    sie = pick<NM>(b.sie, m);
+    u = pick<NM>(b.u, m);
+    rhobar = pick<NM>(b.rhobar, m);
+    res[0] = b.res[0];
+    res[1] = b.res[1];
+    vfrac_total = b.vfrac_total;
+    uscale = b.uscale;
+    utotal_scale = b.utotal_scale;
+    Tnorm = b.Tnorm;
+    Pequil = b.Pequil;
+    Tequil = b.Tequil;
+    err = b.err;
+  }
+  // every wave's values, readable as sh->x[buf][i][k] until the exchange
+  // after the next one
+  __device__ __forceinline__ int Exchange(Real a0, Real a1, Real a2, Real a3) {
+    const int b = turn;
+    turn ^= 1;
+    sh->x[b][0][m] = a0;
+    sh->x[b][1][m] = a1;
+    sh->x[b][2][m] = a2;
+    sh->x[b][3][m] = a3;
+    __syncthreads();
+    return b;
+  }
+  __device__ __forceinline__ void Residual() {
+    const int b = Exchange(vfrac, u, 0.0, 0.0);
+    NeumaierSum sv, se;
+#pragma unroll
+    for (int k = 0; k < NM; ++k) sv.add(sh->x[b][0][k]);
+#pragma unroll
+    for (int k = 0; k < NM; ++k) se.add(sh->x[b][1][k]);
+    res[0] = vfrac_total - sv.result();
+    res[1] = utotal_scale - se.result();
+  }
+  __device__ __forceinline__ void Fixup() {}
+  __device__ __forceinline__ void CheckPTE(bool &conv, bool &ok) const {
+    const Real ev = fabs(res[0]), eu = fabs(res[1]);
+    conv = (ev < P.pte_rel_tolerance_v) && (eu < P.pte_rel_tolerance_e);
+    ok = (eu < P.pte_rel_tolerance_e_sufficient) && (ev < P.pte_rel_tolerance_v_sufficient);
+  }
+  // the two inversions through one call site
+  __device__ __forceinline__ void Jacobian() {
+    Real dudT = 0.0, dudP = 0.0, rbT = 0.0, rbP = 0.0;
+    const Real dp = -Pequil * P.derivative_eps;
+    const Real dT = Tequil * P.derivative_eps;
+    Real r_pert = rho;
+    Real e_pert = sie;
+    Real t[4] = {0, 0, 0, 0};
+#pragma clang loop unroll(disable)
+    for (int k = 0; k < 2; ++k) {
+      const Real Pk = k == 0 ? uscale * (Pequil + dp) : uscale * Pequil;
+      const Real Tk = k == 0 ? Tnorm * Tequil : Tnorm * (Tequil + dT);
+      const Real dk = k == 0 ? dp : dT;
+      Ev::rhoe_PT(E(m), Pk, Tk, r_pert, e_pert, lam, err);
+      const Real dr = robust::ratio(r_pert - rho, dk);
+      const Real du = robust::ratio(robust::ratio(rhobar * e_pert, uscale) - u, dk);
+      const Real rb = robust::ratio(rhobar, rho * rho) * dr;
+      t[0] = k == 0 ? rb : t[0];
+      t[1] = k == 0 ? du : t[1];
+      t[2] = rb;
+      t[3] = du;
+    }
+    const int b = Exchange(t[0], t[1], t[2], t[3]);
+#pragma unroll
+    for (int k = 0; k < NM; ++k) {
+      rbP += sh->x[b][0][k];
+      dudP += sh->x[b][1][k];
+      rbT += sh->x[b][2][k];
+      dudT += sh->x[b][3][k];
+    }
+    jac[0] = -rbT;
+    jac[1] = -rbP;
+    jac[2] = dudT;
+    jac[3] = dudP;
+  }
+  __device__ __forceinline__ bool Solve() {
+    dx[0] = res[0];
+    dx[1] = res[1];
+    return solve_small<2>(jac, dx);
+  }
+  __device__ __forceinline__ Real ScaleDx() {
+    Real scale = 1.0;
+    if (scale * dx[0] < -0.95 * Tequil) scale = robust::ratio(-0.95 * Tequil, dx[0]);
+    const Real own =
+        fabs(0.95 * robust::ratio(robust::ratio(Ev::min_pressure(E(m)), uscale) - Pequil, dx[1]));
+    const int b = Exchange(own, 0.0, 0.0, 0.0);
+#pragma unroll
+    for (int k = 0; k < NM; ++k) scale = smin(fabs(scale), sh->x[b][0][k]);
+    // each bound's temperature follows from the scale so far
+#pragma clang loop unroll(disable)
+    for (int k = 0; k < NM; ++k) {
+      const Real Ttest = (Tequil + scale * dx[0]) * Tnorm;
+      int ek = eidx[0];
+#pragma unroll
+      for (int q = 1; q < NM; ++q) ek = k == q ? (int)eidx[q] : ek;
+      const Real Pmax = Ev::max_pressure_at_T(registry_entry(ek), Ttest, err);
+      scale = smin(fabs(scale),
+                   fabs(0.95 * robust::ratio(robust::ratio(Pmax, uscale) - Pequil, dx[0])));
+    }
+    dx[0] *= scale;
+    dx[1] *= scale;
+    return scale;
+  }
+  __device__ __forceinline__ Real TestUpdate(Real scale, bool cache_state) {
+    if (cache_state) {
+      Ttemp = Tequil;
+      Ptemp = Pequil;
+    }
+    Tequil = Ttemp + scale * dx[0];
+    Pequil = Ptemp + scale * dx[1];
+    Ev::rhoe_PT(E(m), Pequil * uscale, Tequil * Tnorm, rho, sie, lam, err);
+    vfrac = robust::ratio(rhobar, rho);
+    u = robust::ratio(sie * rhobar, uscale);
+    Residual();
+    NeumaierSum s;
+    s.add(res[0] * res[0]);
+    s.add(res[1] * res[1]);
+    return 0.5 * s.result();
+  }
+  // the state that lives from pass to pass: this wave's words and the cell's
+  // (vfrac, u and the residual follow from them)
+  struct Copy {
+    Real rho, sie, lRho, lT, P, T;
+    int err, small, maxline;
+  };
+  __device__ __forceinline__ Copy State(const DriverState &d) const {
+    return Copy{rho, sie, lam.lRho, lam.lT, Pequil, Tequil, err, d.small_step_iters,
+                d.max_line_niter};
+  }
+  // whether every wave finds its words unchanged
+  __device__ __forceinline__ bool Same(const Copy &a, const Copy &c) {
+    auto eq = [](Real x, Real y) {
+      return __builtin_bit_cast(unsigned long long, x) == __builtin_bit_cast(unsigned long long, y);
+    };
+    const bool s = eq(a.rho, c.rho) && eq(a.sie, c.sie) && eq(a.lRho, c.lRho) &&
+                   eq(a.lT, c.lT) && eq(a.P, c.P) && eq(a.T, c.T) && a.err == c.err &&
+                   a.small == c.small && a.maxline == c.maxline;
+    const int b = Exchange(s ? 1.0 : 0.0, 0.0, 0.0, 0.0);
+    bool all = true;
+#pragma unroll
+    for (int k = 0; k < NM; ++k) all = all && sh->x[b][0][k] != 0.0;
+    return all;
+  }
+  // the team's error bits
+  __device__ __forceinline__ int ErrAll() {
+    const int b = Exchange((Real)err, 0.0, 0.0, 0.0);
+    int e = 0;
+#pragma unroll
+    for (int k = 0; k < NM; ++k) e |= (int)sh->x[b][0][k];
+    return e;
+  }
+};
+
 // Whether one TestUpdate's result depends only on the state before the line
 // search and its own scale (so trial steps can run on separate lanes):
 // RhoT, FixedT and FixedP evaluate each material at the trial state; PT's

@@ -363,6 +363,10 @@ constexpr int TailWavesL1() {
   return NM >= 5 ? SGM_TAIL_WAVES_PER_EU_LARGE : 2;
 }
 
+// Parked cells of a PT batch up to which each runs on a workgroup of its own
+// (four cells per CU)
+constexpr int TEAM_MAX = 1024;
+
 // Level 2 of a RhoT tail: the block's one wave takes record items (wave
 // slot, position) from the bin's queue pk.l2_next until none is left, and
 // runs each remaining cell with all 64 lanes (pte_iterate_wide). The
@@ -455,6 +459,7 @@ __device__ __forceinline__ void tail_body(const PteArgs &a, const MixParamsDev &
     const int lpw = one_run && !grp
                         ? min(64, max(1, (claimed + (int)gridDim.x - 1) / (int)gridDim.x))
                         : per_slot;
+    if (METHOD == PTE_PT && one_run && pk.nwaves < 0) return;  // the team kernel's
     const long steps = !one_run ? (pk.nwaves + spb - 1) / spb : (claimed + lpw - 1) / lpw;
     for (long W = blockIdx.x; W < steps; W += gridDim.x) {
       int r = 0, i;
@@ -553,7 +558,11 @@ __device__ __forceinline__ ParkArgs batch_park(const BatchArgs &b) {
   pk.run_base = sm;
   pk.run_cap = sm + 1;
   pk.run_count = sm + 2;
-  pk.nwaves = 0;  // one run: its claimed records
+  // one run: its claimed records; -1 where the batch's parked cells go to the
+  // team kernel
+  int parked = 0;
+  for (int k = 0; k < 5; ++k) parked += b.small[BATCH_SMALL * k + 2];
+  pk.nwaves = parked <= TEAM_MAX ? -1 : 0;
   pk.after2 = b.after2;
   pk.l2_count = sm + 3;
   pk.l2_next = sm + 4;
@@ -602,6 +611,86 @@ pte_batch_tails_kernel(PteArgs a, MixParamsDev P, BatchArgs b, int resident, int
 #undef SGM_ONE
 }
 
+// The parked cells of a PT bin, one per workgroup of NM waves (TeamPT), while
+// the batch parked at most TEAM_MAX; past that one lane per cell has the
+// higher throughput: 400 parked cells (3,001 cells at default tolerances) 134
+// -> 95 ms, 2,700 parked cells 193 -> 225 ms. Every wave of the team takes the same decisions: they follow
+// from values formed alike from the exchanged terms.
+template <int NM>
+__device__ __forceinline__ void team_body(const PteArgs &a, const MixParamsDev &P,
+                                          const ParkArgs &pk) {
+  using Base = SysOf<NM, PTE_PT, false>;
+  __shared__ typename TeamPT<NM>::Shared sh;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if (wave >= NM) return;  // ended waves are not waited for
+  const int claimed = min(pk.run_count[0], pk.run_cap[0]);
+  int turn = 0;
+  for (int W = blockIdx.x; W < claimed; W += gridDim.x) {
+    const long slot = (long)pk.run_base[0] + W;
+    const long c = pk.cell_of[slot];
+    TeamPT<NM> s;
+    DriverState d;
+    CellStatus st;
+    {
+      Base b;
+      ParkLoad(b, d, st, pk.rec + slot * pk.stride);
+      s.Take(b, wave, &sh, turn);
+    }
+    s.P = P;
+    ProbeGate gate;
+    gate.start(d.err);
+    typename TeamPT<NM>::Copy copy = s.State(d);
+    for (;;) {
+      const bool done = pte_step(s, d, st);
+      if (__builtin_amdgcn_readfirstlane(done ? 1 : 0)) break;
+      const bool due = gate.due(d.err);
+      if (__builtin_amdgcn_readfirstlane(due ? 1 : 0)) {
+        const typename TeamPT<NM>::Copy now = s.State(d);
+        if (gate.skip(s.Same(now, copy))) skip_to_last_pass(d);
+        copy = now;
+      }
+    }
+    st.converged = d.converged ? 1 : 0;
+    st.residual = d.err;
+    st.err = s.ErrAll();
+    turn = s.turn;
+    if ((threadIdx.x & 63) == 0) {
+      const long k = a.offsets[c] + wave;
+      a.rho[k] = s.rho;
+      a.vfrac[k] = s.vfrac;
+      a.sie[k] = s.sie;
+      a.temp[k] = s.Tequil * s.Tnorm;
+      a.press[k] = s.Pequil * s.uscale;
+      if (a.lambda) {
+        a.lambda[3L * k + 0] = s.lam.lRho;
+        a.lambda[3L * k + 1] = s.lam.lT;
+      }
+      if (wave == 0) {
+        if (a.conv) a.conv[c] = st.converged;
+        if (a.niter) a.niter[c] = st.niter;
+        if (a.resid) a.resid[c] = st.residual;
+        if (a.err) a.err[c] = st.err;
+      }
+    }
+  }
+}
+template <int METHOD>
+__global__ void __launch_bounds__(64 * 6) pte_batch_team_kernel(PteArgs a, MixParamsDev P,
+                                                                BatchArgs b) {
+  extern __shared__ EosDev lds[];
+  const int nm = BinMaxNM(METHOD) - (int)blockIdx.y;
+  const int *sm = b.small + BATCH_SMALL * (nm - 2);
+  const int claimed = min(sm[2], sm[1]);
+  int parked = 0;
+  for (int k = 0; k < 5; ++k) parked += b.small[BATCH_SMALL * k + 2];
+  if (parked > TEAM_MAX || (int)blockIdx.x >= claimed) return;
+  stage_registry(lds, a.d_eos, a.nreg);
+#define SGM_ONE(K)                                                                             \
+  case K: team_body<K>(a, P, batch_park<K>(b)); break;
+  switch (nm) { SGM_ONE(2) SGM_ONE(3) SGM_ONE(4) SGM_ONE(5) SGM_ONE(6) }
+#undef SGM_ONE
+}
+
 template <int METHOD>
 hipError_t batch_launch(const PteArgs &a, const MixParamsDev &P, const BatchArgs &b,
                         const int *cells, const long *range, long n, int chunk, hipStream_t s) {
@@ -616,6 +705,12 @@ hipError_t batch_launch(const PteArgs &a, const MixParamsDev &P, const BatchArgs
   const int gt = (int)(n < 4L * ncu ? n : 4L * ncu);
   pte_batch_tails_kernel<METHOD, 1><<<dim3(gt, nbin), 64, lds, s>>>(a, P, b, 4 * ncu, 4 * ncu);
   e = hipGetLastError();
+  if constexpr (METHOD == PTE_PT) {
+    if (e != hipSuccess) return e;
+    const int gm = (int)(n < TEAM_MAX ? n : TEAM_MAX);
+    pte_batch_team_kernel<METHOD><<<dim3(gm, nbin), 64 * 6, lds, s>>>(a, P, b);
+    return hipGetLastError();
+  }
   if (e != hipSuccess || TailGroup(METHOD, 2) == 1 || P.line_search_max_iter > TailGroup(METHOD, 2))
     return e;
   pte_batch_tails_kernel<METHOD, 2><<<dim3(gt, nbin), 64, lds, s>>>(a, P, b, 4 * ncu, 4 * ncu);
