@@ -179,17 +179,33 @@ SGM_HD bool regula_falsi(const F &f, Real ytarget, Real guess, Real a, Real b, R
   return it != NITER_MAX;
 }
 
-// secant (:430-510) with a central finite-difference slope
+// f at three points one after another; a function whose evaluation is one
+// long dependent chain passes find_root a form that evaluates them side by
+// side (the functions are pure: the values do not depend on the order)
 template <typename F>
-SGM_HD bool secant(const F &f, Real ytarget, Real xguess, Real xmin, Real xmax, Real xtol,
+struct Three {
+  const F &f;
+  SGM_HD void operator()(const Real (&x)[3], Real (&y)[3]) const {
+    y[0] = f(x[0]);
+    y[1] = f(x[1]);
+    y[2] = f(x[2]);
+  }
+};
+
+// secant (:430-510) with a central finite-difference slope
+template <typename F, typename F3>
+SGM_HD bool secant(const F &f, const F3 &f3, Real ytarget, Real xguess, Real xmin, Real xmax, Real xtol,
                    Real ytol, Real &xroot) {
   Real x = xguess, x_last = xguess;
   for (int iter = 0; iter < NITER_MAX; ++iter) {
     x_last = x;
     const Real dx = fabs(1.e-7 * x) + xtol;
-    const Real y = f(x) - ytarget;
-    const Real yp = f(x + dx);
-    const Real ym = f(x - dx);
+    const Real at[3] = {x, x + dx, x - dx};
+    Real fx[3];
+    f3(at, fx);
+    const Real y = fx[0] - ytarget;
+    const Real yp = fx[1];
+    const Real ym = fx[2];
     const Real dy = (yp - ym) / (2. * dx);
     x -= y / dy;
     if (x < xmin) x = xmin;
@@ -258,9 +274,9 @@ SGM_HD bool bisect(const F &f, Real ytarget, Real xguess, Real xmin, Real xmax, 
 }
 
 // findRoot (:312-373): edge check, secant, then bisection
-template <typename F>
-SGM_HD bool find_root(const F &f, Real ytarget, Real xguess, Real xmin, Real xmax, Real xtol,
-                      Real ytol, Real &xroot) {
+template <typename F, typename F3>
+SGM_HD bool find_root(const F &f, const F3 &f3, Real ytarget, Real xguess, Real xmin, Real xmax,
+                      Real xtol, Real ytol, Real &xroot) {
   const Real fmax = f(xmax);
   if (fabs(fmax - ytarget) / (fabs(fmax) + ytol) < ytol) {
     xroot = xmax;
@@ -273,11 +289,16 @@ SGM_HD bool find_root(const F &f, Real ytarget, Real xguess, Real xmin, Real xma
   }
   if (xguess >= xmax) xguess = xmax - xtol;
   if (xguess <= xmin) xguess = xmin + xtol;
-  if (secant(f, ytarget, xguess, xmin, xmax, xtol, ytol, xroot)) return true;
+  if (secant(f, f3, ytarget, xguess, xmin, xmax, xtol, ytol, xroot)) return true;
   const bool ok = bisect(f, ytarget, xguess, xmin, xmax, xtol, ytol, xroot);
   if (is_nan_or_inf(xroot)) return false;
   if (xroot < xmin || xroot > xmax) return false;
   return ok;
+}
+template <typename F>
+SGM_HD bool find_root(const F &f, Real ytarget, Real xguess, Real xmin, Real xmax, Real xtol,
+                      Real ytol, Real &xroot) {
+  return find_root(f, Three<F>{f}, ytarget, xguess, xmin, xmax, xtol, ytol, xroot);
 }
 } // namespace root
 
@@ -363,6 +384,66 @@ SGM_HD double cbrt(double x) {
   for (int i = 0; i < 5; ++i) y = div3(2.0 * y + mm / (y * y));
   y *= pow2i(q + adj);
   return x < 0 ? -y : y;
+}
+// exp and cbrt of three arguments, the same operations side by side: one is
+// a chain of dependent operations that leaves most issue slots of its wave
+// empty. Arguments off the plain range go through the scalar routines.
+SGM_HD void exp3(const double (&x)[3], double (&y)[3]) {
+  if (!(fabs(x[0]) <= 708.0 && fabs(x[1]) <= 708.0 && fabs(x[2]) <= 708.0)) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) y[i] = exp(x[i]);
+    return;
+  }
+  const double c[13] = {2.08767569878681e-09,  2.505210838544172e-08, 2.755731922398589e-07,
+                        2.7557319223985893e-06, 2.48015873015873e-05, 0.0001984126984126984,
+                        0.001388888888888889,  0.008333333333333333, 0.041666666666666664,
+                        0.16666666666666666,   0.5,                  1.0, 1.0};
+  double kd[3], r[3], p[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    kd[i] = floor(x[i] * 1.4426950408889634 + 0.5);
+    r[i] = (x[i] - kd[i] * 6.93147180369123816490e-01) - kd[i] * 1.90821492927058770002e-10;
+    p[i] = 1.6059043836821613e-10;
+  }
+#pragma unroll
+  for (int k = 0; k < 13; ++k)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) p[i] = p[i] * r[i] + c[k];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) y[i] = p[i] * pow2i((int)kd[i]);
+}
+SGM_HD void cbrt3(const double (&x)[3], double (&y)[3]) {
+  bool plain = true;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    plain = plain && x[i] >= 2.2250738585072014e-308 && x[i] <= 1.7976931348623157e308;
+  if (!plain) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) y[i] = cbrt(x[i]);
+    return;
+  }
+  double mm[3];
+  int q[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const std::int64_t bits = nqt::as_int(x[i]);
+    const int e = (int)((bits >> 52) & 0x7ff) - 1023;
+    const double m = nqt::as_double((bits & nqt::mantissa_mask) | (std::int64_t(1023) << 52));
+    int s = e % 3;
+    q[i] = e / 3;
+    if (s < 0) {
+      s += 3;
+      q[i] -= 1;
+    }
+    mm[i] = s == 0 ? m : (s == 1 ? 2.0 * m : 4.0 * m);
+    y[i] = (-0.011593381976926909 * mm[i] + 0.23742467276201396) * mm[i] + 0.8208312163657417;
+  }
+#pragma unroll
+  for (int k = 0; k < 5; ++k)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) y[i] = div3(2.0 * y[i] + mm[i] / (y[i] * y[i]));
+#pragma unroll
+  for (int i = 0; i < 3; ++i) y[i] *= pow2i(q[i]);
 }
 } // namespace pmath
 
