@@ -277,6 +277,24 @@ SGM_HD Real P_from(const TableDev &t, Real rho, Real lRho, Real T, Real lT, int 
   }
   return bilerp(t, t.P, lRho, lT);
 }
+// sie_from and P_from at one point: on the table one set of weights and all
+// eight loads in flight at once instead of two batches of four
+SGM_HD Real sie_P_from(const TableDev &t, Real rho, Real lRho, Real T, Real lT, int where,
+                       Real &P) {
+  if (where != OnTable) {
+    P = P_from(t, rho, lRho, T, lT, where);
+    return sie_from(t, lRho, T, lT, where);
+  }
+  const W1 wr = grid_weights(lRho, t.lRhoMin, t.dlRho, t.inv_dlRho, t.nRho);
+  const W1 wt = grid_weights(lT, t.lTMin, t.dlT, t.inv_dlT, t.nT);
+  const size_t o = (size_t)wr.ix * t.nT + wt.ix;
+  const Real *e0 = t.sie + o, *p0 = t.P + o;
+  const Real *e1 = e0 + t.nT, *p1 = p0 + t.nT;
+  const Real a0 = e0[0], a1 = e0[1], a2 = e1[0], a3 = e1[1];
+  const Real b0 = p0[0], b1 = p0[1], b2 = p1[0], b3 = p1[1];
+  P = (wr.w0 * (wt.w0 * b0 + wt.w1 * b1) + wr.w1 * (wt.w0 * b2 + wt.w1 * b3));
+  return (wr.w0 * (wt.w0 * a0 + wt.w1 * a1) + wr.w1 * (wt.w0 * a2 + wt.w1 * a3));
+}
 SGM_HD Real cv_from(const TableDev &t, Real lRho, Real lT, int where) {
   Real Cv;
   if (where == OffBottom)
@@ -690,8 +708,8 @@ SGM_HD Real base_e_rT_with_P(const EosDev &e, Real rho, Real T, Lam &lam, Real &
       const Real lRho = table::lRho_(t, r);
       lam.set(lRho, lT);
       const int w = table::loc_rho_T(t, lRho, lT);
-      if (pass == 0) en = table::sie_from(t, lRho, T, lT, w);
-      P_T = table::P_from(t, r, lRho, T, lT, w);
+      const Real e_r = table::sie_P_from(t, r, lRho, T, lT, w, P_T);
+      if (pass == 0) en = e_r;
       if (rhoP == rho) break;
       r = rhoP;
     }

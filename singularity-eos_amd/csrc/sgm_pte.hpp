@@ -850,11 +850,13 @@ struct PteRhoT : PteBase<NM, NM, MODS> {
   // derivatives (t even) or temperature derivatives (t odd), the two fused
   // e/P evaluations of MaterialDerivs, written as one code path so that the
   // wave runs each material kind's evaluation once. Every lane then gathers
-  // the derivatives in material order and each lambda cache from the
-  // temperature lane, whose evaluation MaterialDerivs makes last (the
-  // evaluations write the caches and never read them). The values, the order
-  // of the dedT sum and the caches are those of Jacobian().
-  __device__ __forceinline__ void JacobianWide(int lane) {
+  // the derivatives in material order. The values and the order of the dedT
+  // sum are those of Jacobian(). Returns the lane's lambda cache: the caches
+  // after Jacobian() are those of the temperature lanes, whose evaluation
+  // MaterialDerivs makes last (the evaluations write the caches and never
+  // read them), and only a pass that ends before its first trial needs them
+  // (TakeJacobianLam).
+  __device__ __forceinline__ Lam JacobianWide(int lane) {
     const Real Tcur = Tnorm * Tequil;
     const Real dT = Tequil * P.derivative_eps;
     const Real Tpert = Tnorm * (Tequil + dT);
@@ -890,10 +892,16 @@ struct PteRhoT : PteBase<NM, NM, MODS> {
       dedv[k] = __shfl(de, k, 64);
       dpdT[k] = __shfl(dp, 8 + k, 64);
       dedT_sum += __shfl(de, 8 + k, 64);
+    }
+    AssembleJacobian(dpdv, dedv, dpdT, dedT_sum);
+    return l;
+  }
+  __device__ __forceinline__ void TakeJacobianLam(const Lam &l) {
+#pragma unroll
+    for (int k = 0; k < NM; ++k) {
       lam[k].lRho = __shfl(l.lRho, 8 + k, 64);
       lam[k].lT = __shfl(l.lT, 8 + k, 64);
     }
-    AssembleJacobian(dpdv, dedv, dpdT, dedT_sum);
   }
   SGM_HD void AssembleJacobian(const Real (&dpdv)[NM], const Real (&dedv)[NM],
                                const Real (&dpdT)[NM], Real dedT_sum) {
@@ -985,12 +993,18 @@ struct PteRhoT : PteBase<NM, NM, MODS> {
   }
   // TestUpdate by a whole wave (pte_iterate_wide): lane 8 t + m takes the
   // trial's new temperature and volume fractions like every lane, then
-  // evaluates material m only; the eight lanes of each t then gather the
-  // materials' densities, energies, pressures and lambda caches in material
-  // order and form the residual. Each group of eight lanes can run a trial
-  // of its own scale. The values, the order of every sum and the caches are
-  // those of TestUpdate.
-  __device__ __forceinline__ Real TestUpdateWide(Real scale, bool cache_state, int lane) {
+  // evaluates material m only; the eight lanes of each t gather the pressures
+  // and energies in material order and form the residual. What the residual
+  // does not need (density, energy per mass, lambda cache) stays with its
+  // lane in `own` until a trial is accepted (TakeWide). Each group of eight
+  // lanes can run a trial of its own scale. The values and the order of every
+  // sum are those of TestUpdate.
+  struct OwnTrial {
+    Real rho, sie;
+    Lam lam;
+  };
+  __device__ __forceinline__ Real TestUpdateWide(Real scale, bool cache_state, int lane,
+                                                 OwnTrial &own) {
     if (cache_state) {
       Ttemp = Tequil;
 #pragma unroll
@@ -1028,15 +1042,30 @@ struct PteRhoT : PteBase<NM, NM, MODS> {
     const int b = lane & ~7;
 #pragma unroll
     for (int k = 0; k < NM; ++k) {
-      rho[k] = __shfl(rh, b + k, 64);
-      sie[k] = __shfl(se, b + k, 64);
       u[k] = __shfl(us, b + k, 64);
       press[k] = __shfl(pr, b + k, 64);
-      lam[k].lRho = __shfl(l.lRho, b + k, 64);
-      lam[k].lT = __shfl(l.lT, b + k, 64);
     }
+    own.rho = rh;
+    own.sie = se;
+    own.lam = l;
     Residual();
     return B::ResidualNorm();
+  }
+  // every lane takes the trial of the lanes 8 t .. 8 t + 7
+  __device__ __forceinline__ void TakeWide(const OwnTrial &own, int t) {
+    const int b = 8 * t;
+#pragma unroll
+    for (int k = 0; k < NM; ++k) {
+      rho[k] = __shfl(own.rho, b + k, 64);
+      sie[k] = __shfl(own.sie, b + k, 64);
+      lam[k].lRho = __shfl(own.lam.lRho, b + k, 64);
+      lam[k].lT = __shfl(own.lam.lT, b + k, 64);
+      vfrac[k] = __shfl(vfrac[k], b, 64);
+      u[k] = __shfl(u[k], b, 64);
+      press[k] = __shfl(press[k], b, 64);
+      res[k] = __shfl(res[k], b, 64);
+    }
+    Tequil = __shfl(Tequil, b, 64);
   }
   SGM_HD Real Tout() const { return Tequil * Tnorm; }
   template <class F>
@@ -2340,8 +2369,9 @@ __device__ __forceinline__ bool pte_iterate_wide(S &s, DriverState &d, CellStatu
   st.niter = d.niter;
   s.CheckPTE(d.converged, d.close_enough);
   if (d.converged) return true;
-  s.JacobianWide(lane);
+  const Lam jl = s.JacobianWide(lane);
   if (!s.SolveWave(lane)) {
+    s.TakeJacobianLam(jl);
     d.converged = false;
     s.err |= ERRB_LINSOLVE;
     return true;
@@ -2349,6 +2379,7 @@ __device__ __forceinline__ bool pte_iterate_wide(S &s, DriverState &d, CellStatu
   Real scale = smin(1.0, s.ScaleDx());
   if (fabs(scale) < p.pte_small_step_thresh) d.small_step_iters++;
   if (d.small_step_iters >= p.pte_small_step_tries) {
+    s.TakeJacobianLam(jl);
     d.converged = false;
     s.err |= ERRB_SMALLSTEP;
     return true;
@@ -2356,34 +2387,37 @@ __device__ __forceinline__ bool pte_iterate_wide(S &s, DriverState &d, CellStatu
   const Real gradfdx = -2.0 * scale * d.err;
   const Real err_old = d.err;
   // The two trial stages around one (rolled) TestUpdateWide. Stage 0: the
-  // full step (t = 1: the half step). Stage 1, when the full step does not
-  // decrease the residual enough: lanes of t the t-th scale of the
-  // backtracking loop (scales past line_search_max_iter are computed and
-  // unused; every lane takes part in the gathers).
+  // full step, the half step and, in the lanes past them, the scales of the
+  // backtracking loop that starts from the half step, which is where it
+  // starts unless the half step is the better of the two and its quadratic
+  // fit gives another start; then stage 1 is not needed. Stage 1: lanes of t
+  // the t-th scale from the fitted start (scales past line_search_max_iter
+  // are computed and unused; every lane takes part in the gathers).
   Real err_full = 0, err_mid = 0, sc0 = 0.5;
   bool search = false;
+  int t0 = 1;  // the lanes' t of the loop's first scale
   Real ks[8];
+  typename S::OwnTrial own;
 #pragma clang loop unroll(disable)
   for (int stage = 0; stage < 2; ++stage) {
-    Real sk = t == 1 ? 0.5 : 1.0;
-    if (stage == 1) {
-      sk = sc0;
-      for (int k = 0; k < t; ++k) sk *= p.line_search_fac;
-    }
-    const Real e = s.TestUpdateWide(sk, stage == 0, lane);
-    if (stage == 1) {
+    Real sk = sc0;
+    for (int k = 0; k < t - t0; ++k) sk *= p.line_search_fac;
+    if (stage == 0 && t == 0) sk = 1.0;
+    const Real e = s.TestUpdateWide(sk, stage == 0, lane, own);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) ks[k] = __shfl(e, 8 * k, 64);
-      break;
-    }
+    for (int k = 0; k < 8; ++k) ks[k] = __shfl(e, (8 * (k + t0)) & 63, 64);
+    if (stage == 1) break;
     err_full = __shfl(e, 0, 64);
-    err_mid = __shfl(e, 8, 64);
-    // a scalar: the loop's exit is uniform
+    err_mid = ks[0];
+    // scalars: the loop's exit is uniform
     search = __builtin_amdgcn_readfirstlane(
         err_full > err_old + p.line_search_alpha * gradfdx ? 1 : 0);
-    if (err_mid < err_full && err_mid < err_old)
+    const bool fit = err_mid < err_full && err_mid < err_old;
+    if (fit)
       sc0 = 0.75 + 0.5 * robust::ratio(err_mid - err_full, err_full - 2.0 * err_mid + err_old);
     if (!(search && p.line_search_max_iter > 0)) break;
+    if (!__builtin_amdgcn_readfirstlane(fit || p.line_search_max_iter > 7 ? 1 : 0)) break;
+    t0 = 0;
   }
   int src = 0;
   Real err = err_full;
@@ -2404,13 +2438,13 @@ __device__ __forceinline__ bool pte_iterate_wide(S &s, DriverState &d, CellStatu
           sc *= p.line_search_fac;
         }
       }
-      src = chosen;
+      src = chosen + t0;
       err = pick<8>(ks, chosen);
       const int failed = found ? chosen - 1 : p.line_search_max_iter - 1;
       if (failed > d.max_line_niter) d.max_line_niter = failed;
     }
   }
-  group_take(s, d, st, 8 * src);
+  s.TakeWide(own, src);
   d.err = err;
   s.Fixup();
   if (((err > p.pte_slow_convergence_thresh * err_old) || d.niter == d.max_iter - 1) &&
