@@ -45,8 +45,11 @@ struct TableDev {
   int nRho, nT, reproducible, pad;
   const Real *P, *sie, *bMod, *dEdT, *dPdE;
   const Real *PCold, *sieCold, *bModCold, *dPdECold, *dEdTCold;
-  const Real *PMax, *sielTMax, *dEdTMax, *gm1Max;
+  const Real *sielTMax, *dEdTMax, *gm1Max;
   const Real *rho_at_pmin;
+  // [nRho][nT][4] = {sie, P, dEdT, bMod} of a node: a lookup of several fields
+  // reads two cache lines instead of two a field (device only)
+  const Real *node;
 };
 
 // 288-byte POD describing one material; the closure and vector kernels stage
@@ -179,7 +182,8 @@ struct InvT {
 // call site would grow code that is already instruction-cache bound, and
 // inline in the vector kernels (SGM_TABLE_INVERSE_INLINE), where an
 // out-of-line call would save the callee's registers to scratch memory at
-// every point. Same arithmetic either way.
+// every point. Same arithmetic either way. So do the Gruneisen P-T inversion
+// and maximum density.
 #ifdef SGM_TABLE_INVERSE_INLINE
 #define SGM_TABLE_INV SGM_HD
 #else
@@ -201,8 +205,21 @@ SGM_TABLE_INV InvT lT_from_lRho_sie(const TableDev &t, Real lRho, Real sie, Lam 
     Real lTGuess = t.reproducible ? t.lTMin : 0.5 * (t.lTMin + t.lTMax);
     if (lam.present && (t.lTMin <= lam.lT) && (lam.lT <= t.lTMax)) lTGuess = lam.lT;
     const W1 wr = grid_weights(lRho, t.lRhoMin, t.dlRho, t.inv_dlRho, t.nRho);
-    const Real *sief = t.sie;
-    auto f = [&](Real x) { return bilerp_w(t, sief, wr, x); };
+    // the interval's four values stay in registers: the later steps of a root
+    // find mostly stay in one interval, and a step's loads are what it waits
+    // for (and, over many points, what the caches are busy with)
+    const Real *row = t.sie + (size_t)wr.ix * t.nT;
+    int at = -1;
+    Real v0 = 0, v1 = 0, v2 = 0, v3 = 0;
+    auto f = [&](Real x) {
+      const W1 wt = grid_weights(x, t.lTMin, t.dlT, t.inv_dlT, t.nT);
+      if (wt.ix != at) {
+        at = wt.ix;
+        const Real *r0 = row + at, *r1 = r0 + t.nT;
+        v0 = r0[0], v1 = r0[1], v2 = r1[0], v3 = r1[1];
+      }
+      return (wr.w0 * (wt.w0 * v0 + wt.w1 * v1) + wr.w1 * (wt.w0 * v2 + wt.w1 * v3));
+    };
     if (!root::regula_falsi(f, sie, lTGuess, t.lTMin, t.lTMax, ROOT_THRESH, ROOT_THRESH, lT,
                             &iters))
       lT = t.reproducible ? t.lTMin : lTGuess;
@@ -241,11 +258,16 @@ SGM_TABLE_INV InvRho lRho_from_P_lT(const TableDev &t, Real P, Real lT, Lam lam)
   } else {
     where = OnTable;
     const W1 wt = grid_weights(lT, t.lTMin, t.dlT, t.inv_dlT, t.nT);
+    int at = -1;
+    Real v0 = 0, v1 = 0, v2 = 0, v3 = 0;
     auto f = [&](Real x) {
       const W1 wr = grid_weights(x, t.lRhoMin, t.dlRho, t.inv_dlRho, t.nRho);
-      const Real *r0 = t.P + (size_t)wr.ix * t.nT + wt.ix;
-      const Real *r1 = r0 + t.nT;
-      return (wr.w0 * (wt.w0 * r0[0] + wt.w1 * r0[1]) + wr.w1 * (wt.w0 * r1[0] + wt.w1 * r1[1]));
+      if (wr.ix != at) {
+        at = wr.ix;
+        const Real *r0 = t.P + (size_t)at * t.nT + wt.ix, *r1 = r0 + t.nT;
+        v0 = r0[0], v1 = r0[1], v2 = r1[0], v3 = r1[1];
+      }
+      return (wr.w0 * (wt.w0 * v0 + wt.w1 * v1) + wr.w1 * (wt.w0 * v2 + wt.w1 * v3));
     };
     ok = root::regula_falsi(f, P, lRhoGuess, rhopmin, t.lRhoMax, ROOT_THRESH, ROOT_THRESH, lRho);
   }
@@ -277,23 +299,29 @@ SGM_HD Real P_from(const TableDev &t, Real rho, Real lRho, Real T, Real lT, int 
   }
   return bilerp(t, t.P, lRho, lT);
 }
-// sie_from and P_from at one point: on the table one set of weights and all
-// eight loads in flight at once instead of two batches of four
+struct alignas(16) Pair2 {
+  Real x, y;
+};
+// sie_from and P_from at one point: on the table one set of weights, the four
+// nodes' values in flight at once, from two cache lines
 SGM_HD Real sie_P_from(const TableDev &t, Real rho, Real lRho, Real T, Real lT, int where,
                        Real &P) {
-  if (where != OnTable) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const bool nodes = where == OnTable;
+#else
+  const bool nodes = false;
+#endif
+  if (!nodes) {
     P = P_from(t, rho, lRho, T, lT, where);
     return sie_from(t, lRho, T, lT, where);
   }
   const W1 wr = grid_weights(lRho, t.lRhoMin, t.dlRho, t.inv_dlRho, t.nRho);
   const W1 wt = grid_weights(lT, t.lTMin, t.dlT, t.inv_dlT, t.nT);
-  const size_t o = (size_t)wr.ix * t.nT + wt.ix;
-  const Real *e0 = t.sie + o, *p0 = t.P + o;
-  const Real *e1 = e0 + t.nT, *p1 = p0 + t.nT;
-  const Real a0 = e0[0], a1 = e0[1], a2 = e1[0], a3 = e1[1];
-  const Real b0 = p0[0], b1 = p0[1], b2 = p1[0], b3 = p1[1];
-  P = (wr.w0 * (wt.w0 * b0 + wt.w1 * b1) + wr.w1 * (wt.w0 * b2 + wt.w1 * b3));
-  return (wr.w0 * (wt.w0 * a0 + wt.w1 * a1) + wr.w1 * (wt.w0 * a2 + wt.w1 * a3));
+  const Pair2 *n0 = reinterpret_cast<const Pair2 *>(t.node) + 2 * ((size_t)wr.ix * t.nT + wt.ix);
+  const Pair2 *n1 = n0 + 2 * t.nT;
+  const Pair2 a = n0[0], b = n0[2], c = n1[0], d = n1[2];
+  P = (wr.w0 * (wt.w0 * a.y + wt.w1 * b.y) + wr.w1 * (wt.w0 * c.y + wt.w1 * d.y));
+  return (wr.w0 * (wt.w0 * a.x + wt.w1 * b.x) + wr.w1 * (wt.w0 * c.x + wt.w1 * d.x));
 }
 SGM_HD Real cv_from(const TableDev &t, Real lRho, Real lT, int where) {
   Real Cv;
@@ -520,7 +548,7 @@ SGM_HD Real bmod_rT(const Real *p, Real rho_in, Real T) {
   return bmod_re(p, rho, e_rT(p, rho, T));
 }
 // :423-477
-SGM_NOINL Real max_stable_density(const Real *p, Real T, int &err) {
+SGM_TABLE_INV Real max_stable_density(const Real *p, Real T, int &err) {
   const Real rho_max = p[10], rho0 = p[6];
   const Real slope_at_max = dPres_drho_e(p, rho_max, e_rT(p, rho_max, T));
   const Real slope_at_ref = dPres_drho_e(p, rho0, e_rT(p, rho0, T));
@@ -537,7 +565,7 @@ SGM_NOINL Real max_stable_density(const Real *p, Real T, int &err) {
   return r;
 }
 // :478-526
-SGM_NOINL void rhoe_PT(const Real *p, Real P, Real T, Real &rho, Real &sie, int &err) {
+SGM_TABLE_INV void rhoe_PT(const Real *p, Real P, Real T, Real &rho, Real &sie, int &err) {
   const Real rho0 = p[6];
   const Real Pref = P_rT(p, rho0, T);
   Real lo, hi, guess, p_used = P;
@@ -1002,10 +1030,43 @@ SGM_HD void fill_table(const EosDev &e, Real &rho, Real &temp, Real &sie, Real &
     lT = table::lT_(t, temp);
   }
   w = table::loc_rho_T(t, lRho, lT);
-  if (output & specific_internal_energy) sie = table::sie_from(t, lRho, temp, lT, w);
-  if (output & pressure) press = table::P_from(t, rho, lRho, temp, lT, w);
-  if (output & specific_heat) cv = table::cv_from(t, lRho, lT, w);
-  if (output & bulk_modulus) bmod = table::bmod_from(t, rho, lRho, temp, lT, w);
+#if defined(__HIP_DEVICE_COMPILE__)
+  const bool nodes = w == table::OnTable;
+#else
+  const bool nodes = false;
+#endif
+  if (nodes) {
+    // the four nodes' records, {sie, P} and {dEdT, bMod} apart (the vector
+    // FillEos was bound by the cache lines of its four separate fields)
+    const W1 wr = grid_weights(lRho, t.lRhoMin, t.dlRho, t.inv_dlRho, t.nRho);
+    const W1 wt = grid_weights(lT, t.lTMin, t.dlT, t.inv_dlT, t.nT);
+    const table::Pair2 *n0 = reinterpret_cast<const table::Pair2 *>(t.node) +
+                             2 * ((size_t)wr.ix * t.nT + wt.ix);
+    const table::Pair2 *n1 = n0 + 2 * t.nT;
+    auto mix = [&](Real a, Real b, Real c, Real d) {
+      return (wr.w0 * (wt.w0 * a + wt.w1 * b) + wr.w1 * (wt.w0 * c + wt.w1 * d));
+    };
+    const bool ep = (output & (specific_internal_energy | pressure)) != 0;
+    const bool cb = (output & (specific_heat | bulk_modulus)) != 0;
+    table::Pair2 ea{}, eb{}, ec{}, ed{}, ca{}, cbp{}, cc{}, cd{};
+    if (ep) ea = n0[0], eb = n0[2], ec = n1[0], ed = n1[2];
+    if (cb) ca = n0[1], cbp = n0[3], cc = n1[1], cd = n1[3];
+    if (output & specific_internal_energy) sie = mix(ea.x, eb.x, ec.x, ed.x);
+    if (output & pressure) press = mix(ea.y, eb.y, ec.y, ed.y);
+    if (output & specific_heat) {
+      const Real c = mix(ca.x, cbp.x, cc.x, cd.x);
+      cv = c > robust::EPS() ? c : robust::EPS();
+    }
+    if (output & bulk_modulus) {
+      const Real b = mix(ca.y, cbp.y, cc.y, cd.y);
+      bmod = b > robust::EPS() ? b : robust::EPS();
+    }
+  } else {
+    if (output & specific_internal_energy) sie = table::sie_from(t, lRho, temp, lT, w);
+    if (output & pressure) press = table::P_from(t, rho, lRho, temp, lT, w);
+    if (output & specific_heat) cv = table::cv_from(t, lRho, lT, w);
+    if (output & bulk_modulus) bmod = table::bmod_from(t, rho, lRho, temp, lT, w);
+  }
   lam.set(lRho, lT);
 }
 SGM_HD void base_fill(const EosDev &e, Real &rho, Real &temp, Real &sie, Real &press, Real &cv,

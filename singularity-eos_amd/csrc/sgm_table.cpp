@@ -26,7 +26,6 @@ void fill_view(TableHost &T) {
   d.bModCold = T.bModCold.data();
   d.dPdECold = T.dPdECold.data();
   d.dEdTCold = T.dEdTCold.data();
-  d.PMax = T.PMax.data();
   d.sielTMax = T.sielTMax.data();
   d.dEdTMax = T.dEdTMax.data();
   d.gm1Max = T.gm1Max.data();
@@ -190,6 +189,16 @@ bool build_table_host(const sgm_table_desc &in, TableHost &T) {
   return true;
 }
 
+__global__ void node_kernel(const Real *sie, const Real *P, const Real *dEdT, const Real *bMod,
+                            size_t n, Real *node) {
+  const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  node[4 * k] = sie[k];
+  node[4 * k + 1] = P[k];
+  node[4 * k + 2] = dEdT[k];
+  node[4 * k + 3] = bMod[k];
+}
+
 // Copies every field to device memory and builds the device TableDev.
 hipError_t upload_table(TableHost &T) {
   TableDev dd = T.hdev;
@@ -215,13 +224,21 @@ hipError_t upload_table(TableHost &T) {
   SGM_UP(bModCold)
   SGM_UP(dPdECold)
   SGM_UP(dEdTCold)
-  SGM_UP(PMax)
   SGM_UP(sielTMax)
   SGM_UP(dEdTMax)
   SGM_UP(gm1Max)
   SGM_UP(rho_at_pmin)
 #undef SGM_UP
   void *p = nullptr;
+  const size_t n2 = T.sie.size();
+  if ((e = hipMalloc(&p, 4 * n2 * sizeof(Real))) != hipSuccess) return e;
+  T.d_arrays.push_back(p);
+  node_kernel<<<(unsigned)((n2 + 255) / 256), 256>>>(dd.sie, dd.P, dd.dEdT, dd.bMod, n2,
+                                                     static_cast<Real *>(p));
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  // contexts are used on any stream from here on
+  if ((e = hipStreamSynchronize(nullptr)) != hipSuccess) return e;
+  dd.node = static_cast<const Real *>(p);
   if ((e = hipMalloc(&p, sizeof(TableDev))) != hipSuccess) return e;
   T.d_arrays.push_back(p);
   if ((e = hipMemcpy(p, &dd, sizeof(TableDev), hipMemcpyHostToDevice)) != hipSuccess) return e;

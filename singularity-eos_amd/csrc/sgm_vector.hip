@@ -168,8 +168,16 @@ __global__ void __launch_bounds__(256)
       lam.lT = lp[1];
     }
     int err = 0;
+    // the kind's inversion inline (out of line, as the closures call it, every
+    // kind's kernel held the Gruneisen inversion's call and saved its
+    // registers to scratch at every point)
     Real r = rho[i], s = 0;
-    eos_rhoe_PT(ek, P[i], T[i], r, s, lam, err);
+    base_rhoe_PT(ek, P[i], T[i], r, s, lam, err);
+    if (ek.mods & MOD_SHIFTED) s = s + ek.shift;
+    if (ek.mods & MOD_SCALED) {
+      r = r * ek.inv_scale;
+      s = s * ek.scale;
+    }
     rho[i] = r;
     sie[i] = s;
     if (lp) {
