@@ -279,13 +279,12 @@ std::vector<size_t> bin_order(const sgm_plan *p) {
   return order;
 }
 
-// Plans of up to this many cells launch their bins together (one kernel for
-// all bins, one per tail level: launch_pte_batch_bins): their bins do not
-// fill the GPU one by one. Larger ones overlap each bin's tail with the next
-// bins' kernels. Together against forked: 2^17 cells
-// of get_sg_eos 63 -> 55 ms, plans of 2,517 cells 10.2 -> 4.7 ms, 142,921 14.6 -> 13.1,
-// 2^18 15.5 -> 13.7.
-constexpr long PLAN_MERGED_CELLS = 1L << 18;
+// A plan launches its bins together (one kernel for all bins, one per tail
+// level: launch_pte_batch_bins) unless a launch shape was set for one, or for
+// RhoU, whose cells past four materials have no bin: the bins then keep their
+// own kernels, each bin's tail beside the next bins'.
+// Together against apart: 2^17 cells of get_sg_eos 63 -> 55 ms, plans of 2,517
+// cells 10.2 -> 4.7 ms, 142,921 14.6 -> 13.1, 2^19 17.5 -> 15.3, 2^20 21.9 -> 19.0.
 
 // Records the counter reset and every bin on stream s: the persistent bin
 // kernels one after another on s; with fork streams (graph capture, or a
@@ -296,7 +295,19 @@ hipError_t launch_bins(sgm_plan *p, const PteArgs &a, const MixParamsDev &P, hip
                        bool fork) {
   hipError_t e = reset_counters(p, s);
   if (e != hipSuccess) return e;
-  if (p->ncell <= PLAN_MERGED_CELLS && !p->own_shape && p->d_rec) {
+  if (!p->own_shape && p->d_rec && p->method != PTE_RHOU) {
+    // the list bins beside the batch, each on a stream of its own
+    const bool lists = fork && p->aux.size() >= p->bins.size() &&
+                       p->ev.size() >= 2 * p->bins.size();
+    for (size_t i = 0; i < p->bins.size() && lists; ++i) {
+      const Bin &x = p->bins[i];
+      if (x.nm >= 2 && x.nm <= 6) continue;
+      if ((e = hipEventRecord(p->ev[2 * i], s)) != hipSuccess ||
+          (e = hipStreamWaitEvent(p->aux[i], p->ev[2 * i], 0)) != hipSuccess ||
+          (e = launch_list_bin(p, x, a, P, p->d_sorted + x.start, p->aux[i])) != hipSuccess ||
+          (e = hipEventRecord(p->ev[2 * i + 1], p->aux[i])) != hipSuccess)
+        return e;
+    }
     BatchArgs b;
     b.small = p->d_small;
     b.rec = p->d_rec;
@@ -306,9 +317,12 @@ hipError_t launch_bins(sgm_plan *p, const PteArgs &a, const MixParamsDev &P, hip
     b.after2 = 4;
     e = launch_pte_batch_bins(p->method, a, P, b, p->d_sorted, p->d_range, p->ncell,
                               batch_cells_per_wave(p->ncell, device_cu_count()), s);
-    for (const Bin &x : p->bins)
-      if (e == hipSuccess && (x.nm < 2 || x.nm > 6))
-        e = launch_list_bin(p, x, a, P, p->d_sorted + x.start, s);
+    for (size_t i = 0; i < p->bins.size() && e == hipSuccess; ++i) {
+      const Bin &x = p->bins[i];
+      if (x.nm >= 2 && x.nm <= 6) continue;
+      e = lists ? hipStreamWaitEvent(s, p->ev[2 * i + 1], 0)
+                : launch_list_bin(p, x, a, P, p->d_sorted + x.start, s);
+    }
     return e;
   }
   const std::vector<size_t> order = bin_order(p);
