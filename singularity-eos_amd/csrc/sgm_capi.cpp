@@ -533,13 +533,20 @@ static int pte_common(int method, sgm_ctx *ctx, long ncell, long nnz, const int 
   // sort and some twenty launches, about 0.15 ms, against the plain kernel's
   // lanes held by their waves' slowest cells: 7 to 20 times the time on
   // uneven cells of 100 to 20,000). Two-material cells finish within a few
-  // passes of each other: 65,536 of them take the plain kernel 0.19 ms.
-  if (nnz > 2 * ncell) {
+  // passes of each other. RhoU has no bins past four materials and cells with
+  // modified materials none at all: their list kernel would run behind the
+  // other cells' tails instead of beside them (RhoU, 1,000 uneven cells: 265 ms
+  // plain, 310 to 350 as a batch).
+  const bool binned = method != PTE_RHOU && ctx_mod_mask(ctx) == 0;
+  if (nnz > 2 * ncell && binned) {
     bool taken = false;
     const hipError_t e = launch_pte_batch(ctx, method, a, P, (hipStream_t)stream, taken);
     if (e != hipSuccess) return SGM_E_HIP;
     if (taken) return SGM_OK;
   }
+  // exactly two on average, as in a two-material problem: the pair kernel
+  // takes those cells (the batched kernels' solver, without modifiers)
+  a.skip_pairs = nnz == 2 * ncell && binned && ncell <= 1L << 30;
   const hipError_t e = launch_pte_plain(method, a, P, (hipStream_t)stream);
   return e == hipSuccess ? SGM_OK : SGM_E_HIP;
 }

@@ -35,6 +35,8 @@ struct PteArgs {
   // learned initial guess (batched kernels only): per entry vfrac, per cell T
   const double *guess_vfrac = nullptr, *guess_T = nullptr;
   int *used_guess = nullptr;
+  // the plain kernel leaves cells of two materials to the pair kernel
+  bool skip_pairs = false;
 };
 // Straggler parking for the batched bin kernels: a cell still iterating after
 // `after` Newton iterations is saved (ParkSave, ParkWords(nm, nm + 1) FP64
@@ -134,16 +136,23 @@ constexpr bool TailWide(int method, int nm) { return method == PTE_RHOT && nm >=
                                    int block, int cpw, int grid, const ParkArgs *park,         \
                                    hipStream_t s);                                             \
   hipError_t launch_pte_tail_##name(int nm, const PteArgs &a, const MixParamsDev &P,           \
-                                    const ParkArgs &park, hipStream_t s);                      \
-  hipError_t launch_pte_batch_##name(const PteArgs &a, const MixParamsDev &P,                  \
-                                     const BatchArgs &b, const int *cells, const long *range,  \
-                                     long n, int chunk, hipStream_t s);
+                                    const ParkArgs &park, hipStream_t s);
 SGM_PTE_LAUNCHERS(rhot)
 SGM_PTE_LAUNCHERS(pt)
 SGM_PTE_LAUNCHERS(fixedt)
 SGM_PTE_LAUNCHERS(fixedp)
 SGM_PTE_LAUNCHERS(rhou)
 #undef SGM_PTE_LAUNCHERS
+// the bins and tails of a batch (the methods whose bins reach six materials)
+#define SGM_PTE_BATCH(name)                                                                    \
+  hipError_t launch_pte_batch_##name(const PteArgs &a, const MixParamsDev &P,                  \
+                                     const BatchArgs &b, const int *cells, const long *range,  \
+                                     long n, int chunk, hipStream_t s);
+SGM_PTE_BATCH(rhot)
+SGM_PTE_BATCH(pt)
+SGM_PTE_BATCH(fixedt)
+SGM_PTE_BATCH(fixedp)
+#undef SGM_PTE_BATCH
 
 // the plain per-call kernels: one lane per cell of 1..8 materials, one wave
 // per cell of 9..64
@@ -230,7 +239,6 @@ inline hipError_t launch_pte_batch_bins(int method, const PteArgs &a, const MixP
   case PTE_PT: return launch_pte_batch_pt(a, P, b, cells, range, n, chunk, s);
   case PTE_FIXED_T: return launch_pte_batch_fixedt(a, P, b, cells, range, n, chunk, s);
   case PTE_FIXED_P: return launch_pte_batch_fixedp(a, P, b, cells, range, n, chunk, s);
-  case PTE_RHOU: return launch_pte_batch_rhou(a, P, b, cells, range, n, chunk, s);
   default: return hipErrorInvalidValue;
   }
 }

@@ -11,9 +11,4 @@ hipError_t launch_pte_tail_rhou(int nm, const PteArgs &a, const MixParamsDev &P,
                                 const ParkArgs &park, hipStream_t s) {
   return kern::tail_launch<PTE_RHOU>(nm, a, P, park, s);
 }
-hipError_t launch_pte_batch_rhou(const PteArgs &a, const MixParamsDev &P, const BatchArgs &b,
-                               const int *cells, const long *range, long n, int chunk,
-                               hipStream_t s) {
-  return kern::batch_launch<PTE_RHOU>(a, P, b, cells, range, n, chunk, s);
-}
 } // namespace sgm

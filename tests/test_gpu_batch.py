@@ -3,8 +3,10 @@ device, binned kernels with parking and tails, work arrays of the context)
 that calls with more than two materials per cell on average take, and the
 plain kernels, which the same call takes while its stream is being captured.
 Same cells, same bits, at the sizes where the batch changes its lanes per
-wave, with pure, malformed and modified cells among them, and from several
-streams at once (more than the context has workspaces)."""
+wave, with pure and malformed cells among them, and from several streams at
+once (more than the context has workspaces). And the pair kernel that takes
+the two-material cells of calls with exactly two materials on average,
+against the same cells in a call of another average."""
 import numpy as np
 import pytest
 
@@ -90,12 +92,10 @@ def captured(torch, ctx, call):
 
 
 @pytest.mark.parametrize("method,n", [(0, 1), (0, 5), (0, 64), (0, 65), (0, 4097), (0, 20000),
-                                      (1, 300), (2, 1500), (3, 300), (4, 200)])
+                                      (1, 300), (2, 1500), (3, 300)])
 def test_batch_matches_plain_kernels(sgm, workloads, torch_gpu, method, n):
     torch = torch_gpu
     ctx, _ = workloads.pool_context()
-    if n == 1500:
-        ctx.set_modifiers(4, shifted=True, shift=1e8)
     a = cells(workloads, ctx, n, 0x5EED0000 + 900 + n + method, pure=n > 5)
     assert a["nnz"] > 2 * n
     call = Call(torch, sgm, a, method, tight=method == 0)
@@ -124,4 +124,48 @@ def test_batches_from_several_streams(sgm, workloads, torch_gpu):
         torch.cuda.synchronize()
         for c, w in zip(calls, want):
             assert same(c.result(), w)
+    ctx.close()
+
+
+@pytest.mark.parametrize("method,n", [(0, 1), (0, 63), (0, 130), (0, 140001), (1, 64), (2, 65),
+                                      (3, 64), (4, 64)])
+def test_pair_kernel_matches_plain_kernel(sgm, workloads, torch_gpu, method, n):
+    """n gas / stiffened-gas cells alone (the pair kernel; 140,001 cells: waves
+    that stride twice), and behind one pure cell (nnz != 2 ncell: the plain
+    kernel). A call of one pure, one three-material and two-material cells also
+    averages two: the pair kernel leaves the other counts to the plain one."""
+    torch = torch_gpu
+    ctx = sgm.Context(2)
+    ctx.set_ideal(0, *workloads.IDEAL_A)
+    ctx.set_stiff(1, *workloads.STIFF_B)
+    a = workloads.pte2(n, seed=0x5EED0000 + 990 + n)
+    alone = Call(torch, sgm, a, method, tight=False)
+    alone.run(ctx, 0)
+    torch.cuda.synchronize()
+    got = alone.result()
+
+    def front(a, ids):
+        b = dict(a)
+        for k in FIELDS:
+            b[k] = np.concatenate([a[k][:1].repeat(len(ids)), a[k]])
+        b["mat_ids"] = np.concatenate([np.array(ids, np.uint8), a["mat_ids"]])
+        b["offsets"] = np.concatenate([[0], a["offsets"] + len(ids)]).astype(np.int32)
+        for k in ("vfrac_tot", "sie_tot"):
+            b[k] = np.concatenate([a[k][:1], a[k]])
+        b["ncell"], b["nnz"] = a["ncell"] + 1, a["nnz"] + len(ids)
+        return b
+
+    one = front(a, [0])
+    plain = Call(torch, sgm, one, method, tight=False)
+    plain.run(ctx, 0)
+    torch.cuda.synchronize()
+    ref = plain.result()
+    cut = {k: v[1:] for k, v in ref.items()}
+    assert same(got, cut)
+    mixed = Call(torch, sgm, front(one, [0, 1, 0]), method, tight=False)
+    assert mixed.nnz == 2 * mixed.n
+    mixed.run(ctx, 0)
+    torch.cuda.synchronize()
+    m = mixed.result()
+    assert same({k: v[3 if k in FIELDS else 1:] for k, v in m.items()}, ref)
     ctx.close()
