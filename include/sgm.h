@@ -184,7 +184,7 @@ int sgm_vec_rhoe_from_PT(sgm_ctx *ctx, int matindex, const double *P, const doub
                          int *errs, sgm_stream_t stream);
 
 /* ---- PTE closure (plain per-call path) ----------------------------------- */
-/* One launch over a CSR list of mixed cells: cell c owns entries
+/* One call over a CSR list of mixed cells: cell c owns entries
  * [offsets[c], offsets[c+1]) of the per-(cell,material) arrays; mat_ids holds
  * context material indices; 1..64 materials per cell (1..8 one lane per cell
  * with the state in registers, 9..64 one wave per cell with the Newton system
@@ -196,7 +196,14 @@ int sgm_vec_rhoe_from_PT(sgm_ctx *ctx, int matindex, const double *P, const doub
  * Inputs: rho, vfrac (guess), temp and press (guesses; press used by
  * pressure-preferring EOS), vfrac_tot[c], sie_tot[c], Tnorm[c] (NULL = 0).
  * Outputs overwrite rho, vfrac, sie, temp, press. lambda: NULL or [nnz*3].
- * params: HOST pointer (NULL = defaults). */
+ * params: HOST pointer (NULL = defaults).
+ * Calls with more than two materials per cell on average (no material with
+ * modifiers; not sgm_pte_rhoU) sort their cells on the device first, in work
+ * arrays the context keeps between calls (about 0.8 KB per cell of the
+ * largest call, at most 2^20 cells' worth and at most four sets, for calls
+ * that overlap on several streams; sgm_finalize frees them). While the stream
+ * is being captured, or when there is no memory for them, the call runs on
+ * kernels that need none. The results are the same. */
 int sgm_pte_rhoT(sgm_ctx *ctx, long ncell, long nnz, const int *offsets, const uint8_t *mat_ids,
                  double *rho, double *vfrac, double *sie, double *temp, double *press,
                  const double *vfrac_tot, const double *sie_tot, const double *Tnorm,
@@ -320,7 +327,7 @@ int sgm_get_sg_eos_noalloc(sgm_ctx *ctx, int nmat, int ncell, int cell_dim, int 
                            sgm_stream_t stream);
 /* No reference counterpart: frees the work buffers and the batched plan that
  * sgm_get_sg_eos keeps in the context between calls (for the 2^20-cell
- * uneven workload about 0.5 GB of straggler records plus the arenas); the
+ * uneven workload about 0.8 GB of straggler records plus the arenas); the
  * next call rebuilds them. This memory is outside any server's
  * hbm_budget_bytes. sgm_finalize releases it too. */
 int sgm_release_driver_cache(sgm_ctx *ctx);
