@@ -153,6 +153,16 @@ hipError_t launch_batch(int method, const PteArgs &a, const MixParamsDev &P,
   return e != hipSuccess ? e : enqueue(method, a, P, mod_mask, nrec, L, buf, s);
 }
 
+namespace {
+// allocation and event queries of this call stay out of a capture that the
+// same thread holds open on another stream
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+} // namespace
+
 hipError_t launch_pte_batch(sgm_ctx *ctx, int method, const PteArgs &a, const MixParamsDev &P,
                             hipStream_t s, bool &taken) {
   taken = false;
@@ -161,6 +171,7 @@ hipError_t launch_pte_batch(sgm_ctx *ctx, int method, const PteArgs &a, const Mi
     (void)hipGetLastError();
     return hipSuccess;
   }
+  const RelaxedCapture relaxed;
   const long chunk = std::min<long>(a.ncell, BATCH_MAX_CELLS);
   Layout L;
   if (layout(method, chunk, 0, L) != hipSuccess) return hipSuccess;

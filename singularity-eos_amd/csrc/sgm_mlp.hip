@@ -107,6 +107,18 @@ __device__ __forceinline__ void w_store(const u4 (&r)[N], bf16 *dst, int ld) {
     *reinterpret_cast<u4 *>(dst + (c / (COLS / 8)) * ld + (c % (COLS / 8)) * 8) = r[i];
   }
 }
+// 16 features of a row: two 16-byte loads, or, where the caller's matrix is not
+// on a 16-byte boundary, one by one
+__device__ __forceinline__ void load_features(const bf16 *p, bool aligned, u4 (&x)[2]) {
+  if (aligned) {
+    x[0] = reinterpret_cast<const u4 *>(p)[0];
+    x[1] = reinterpret_cast<const u4 *>(p)[1];
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    x[i >> 2][i & 3] = (unsigned)p[2 * i] | ((unsigned)p[2 * i + 1] << 16);
+}
 template <int N>
 __device__ __forceinline__ void zero_acc(f4 (&acc)[N]) {
 #pragma unroll
@@ -198,14 +210,11 @@ __global__ void __launch_bounds__(512, 1) fwd_kernel(const bf16 *__restrict__ wq
   __shared__ InferLds L;
   infer_stage(L, wq);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const bool aligned = (reinterpret_cast<uintptr_t>(Xall) & 15) == 0;
   for (long t = (long)blockIdx.x * 8 + w; t * 16 < B; t += (long)gridDim.x * 8) {
     const long r = t * 16 + (l >> 2);
     u4 x[2] = {u4{0, 0, 0, 0}, u4{0, 0, 0, 0}};
-    if (r < B) {
-      const u4 *src = reinterpret_cast<const u4 *>(Xall + (long)idx[r] * KIN) + (l & 3) * 2;
-      x[0] = src[0];
-      x[1] = src[1];
-    }
+    if (r < B) load_features(Xall + (long)idx[r] * KIN + (l & 3) * 16, aligned, x);
     u4 *d = reinterpret_cast<u4 *>(L.row + (w * 16 + (l >> 2)) * LDH + (l & 3) * 16);
     d[0] = x[0];
     d[1] = x[1];
@@ -310,6 +319,7 @@ __global__ void __launch_bounds__(256, 1)
                  float wT, float inv_b, float *__restrict__ part, float *__restrict__ loss) {
   __shared__ TrainLds L;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, rb = w * 16;
+  const bool aligned = (reinterpret_cast<uintptr_t>(Xall) & 15) == 0;
   bf16 *row = L.row + rb * LDH;
   f4 dw1[2][KIN / 16], dw2[2][H / 16], dw3[2][H / 16], dw4[2];
   float db1[H / 16], db2[H / 16], db3[H / 16], db4 = 0.f;
@@ -336,11 +346,7 @@ __global__ void __launch_bounds__(256, 1)
         bf16 h[16];
       } x;
       x.v[0] = x.v[1] = u4{0, 0, 0, 0};
-      if (r < nrow) {
-        const u4 *src = reinterpret_cast<const u4 *>(Xall + (long)idx[row0 + r] * KIN + q);
-        x.v[0] = src[0];
-        x.v[1] = src[1];
-      }
+      if (r < nrow) load_features(Xall + (long)idx[row0 + r] * KIN + q, aligned, x.v);
       u4 *d = reinterpret_cast<u4 *>(L.row + r * LDH + q);
       d[0] = x.v[0];
       d[1] = x.v[1];

@@ -78,6 +78,14 @@ def test_row_tiles_match_fp64_reference(torch_gpu, L, ref, B):
         gr += gk * sel.sum() * k / B
     # bf16 gradients into the products: 2^-9 per element
     assert np.linalg.norm(g - gr) < 0.03 * np.linalg.norm(gr)
+    # the same features off a 16-byte boundary
+    off = torch.zeros(X.numel() + 1, dtype=torch.int16, device="cuda")
+    off[1:] = X.flatten()
+    X1 = off[1:].view(n, 64)
+    g1, loss1 = mlp.gradients(torch, X1, tgt, idx)
+    assert torch.equal(g1, torch.as_tensor(g, dtype=torch.float32, device="cuda"))
+    assert torch.equal(loss1, loss)
+    assert np.array_equal(mlp.forward(torch, X1, idx).cpu().numpy(), Y)
     mlp.close()
 
 
