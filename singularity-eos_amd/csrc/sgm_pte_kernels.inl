@@ -10,7 +10,12 @@
 //    cells that all have NM materials (sorted by material signature so the
 //    EOS dispatch is wave-uniform); lanes retire finished cells and take new
 //    ones between Newton iterations, from a per-wave reserve refilled
-//    `chunk` (>= 64) cells at a time from a device counter.
+//    `chunk` cells at a time from a device counter (fewer than 64: the lanes
+//    past them stay idle).
+//  * pte_batch_bins_kernel / pte_batch_tails_kernel: all bins of a batch, and
+//    their parked cells, in one launch per stage; pte_batch_team_kernel: the
+//    parked PT cells of a small batch on teams of waves.
+//  * pte_pair_kernel: the two-material cells of a plain call.
 //  * pte_wave_kernel: cells of 9..64 materials, one wave per cell
 //    (sgm_pte_wave.hpp), after the plain kernel and beside the list kernel.
 //
