@@ -26,7 +26,7 @@ int batch_cells_per_wave(long ncell, int ncu) {
 
 namespace {
 
-constexpr int NBIN = 5, NSMALL = BATCH_SMALL;  // bins: material counts 2..6
+constexpr int NBIN = BATCH_BINS;  // material counts 2..6
 constexpr int BATCH_PARK_AFTER = 20, BATCH_AFTER2 = 4;  // as plans
 
 // From the sorted keys: per material count 2..6 {start, count} and the bin's
@@ -35,7 +35,7 @@ constexpr int BATCH_PARK_AFTER = 20, BATCH_AFTER2 = 4;  // as plans
 // range 6 those past the register-resident counts.
 __global__ void batch_tables_kernel(const unsigned long long *__restrict__ keys, long n,
                                     int max_nm, int nrec, long *__restrict__ range,
-                                    int *__restrict__ small) {
+                                    BatchBin *__restrict__ bins) {
   __shared__ long pos[NBIN + 1];  // first position with a count of at least k + 2
   const int t = threadIdx.x;
   if (t <= NBIN) {
@@ -55,10 +55,9 @@ __global__ void batch_tables_kernel(const unsigned long long *__restrict__ keys,
     const long start = pos[t], count = pos[t + 1] - start;
     range[2 * (t + 1)] = start;
     range[2 * (t + 1) + 1] = count;
-    int *s = small + NSMALL * t;
-    s[0] = nrec ? t * nrec : (int)start;
-    s[1] = nrec ? nrec : (int)count;
-    s[2] = s[3] = s[4] = s[5] = 0;
+    bins[t].first = nrec ? t * nrec : (int)start;
+    bins[t].records = nrec ? nrec : (int)count;
+    bins[t].claimed = bins[t].next = bins[t].l2_count = bins[t].l2_next = 0;
   } else if (t == NBIN) {
     range[0] = 0;
     range[1] = pos[0];
@@ -68,7 +67,7 @@ __global__ void batch_tables_kernel(const unsigned long long *__restrict__ keys,
 }
 
 struct Layout {
-  size_t keys, keys2, ids, sorted, range, small, cell_of, rec, tmp, tmp_bytes, total;
+  size_t keys, keys2, ids, sorted, range, bins, cell_of, rec, tmp, tmp_bytes, total;
 };
 // nrec: straggler records per bin; 0: one per cell
 hipError_t layout(int method, long n, int nrec, Layout &L) {
@@ -83,7 +82,7 @@ hipError_t layout(int method, long n, int nrec, Layout &L) {
   L.ids = take(4 * (size_t)n);
   L.sorted = take(4 * (size_t)n);
   L.range = take(sizeof(long) * 2 * (NBIN + 2));
-  L.small = take(sizeof(int) * NSMALL * NBIN);
+  L.bins = take(sizeof(BatchBin) * NBIN);
   const size_t recs = nrec ? (size_t)NBIN * nrec : (size_t)n;
   L.cell_of = take(4 * recs);
   L.rec = take(8 * (size_t)ParkStride(method, BinMaxNM(method)) * recs);
@@ -105,7 +104,7 @@ hipError_t enqueue(int method, const PteArgs &a, const MixParamsDev &P,
   auto *keys2 = (unsigned long long *)(base + L.keys2);
   int *ids = (int *)(base + L.ids), *sorted = (int *)(base + L.sorted);
   long *range = (long *)(base + L.range);
-  int *small = (int *)(base + L.small);
+  auto *bins = (BatchBin *)(base + L.bins);
   const int n = (int)a.ncell;
   const int max_nm = BinMaxNM(method);
   hipError_t e =
@@ -114,10 +113,10 @@ hipError_t enqueue(int method, const PteArgs &a, const MixParamsDev &P,
   size_t tb = L.tmp_bytes;
   e = hipcub::DeviceRadixSort::SortPairs(base + L.tmp, tb, keys, keys2, ids, sorted, n, 0, 64, s);
   if (e != hipSuccess) return e;
-  batch_tables_kernel<<<1, 64, 0, s>>>(keys2, n, max_nm, nrec, range, small);
+  batch_tables_kernel<<<1, 64, 0, s>>>(keys2, n, max_nm, nrec, range, bins);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   BatchArgs b;
-  b.small = small;
+  b.bins = bins;
   b.rec = (double *)(base + L.rec);
   b.cell_of = (int *)(base + L.cell_of);
   b.stride = ParkStride(method, max_nm);

@@ -54,7 +54,8 @@ struct sgm_plan {
   // whose bins share one kernel (BatchArgs): per material count its first
   // record, records, and the counters of the last execution
   double *d_rec = nullptr;
-  int *d_cell_of = nullptr, *d_small = nullptr;
+  int *d_cell_of = nullptr;
+  BatchBin *d_batch = nullptr;
   long *d_range = nullptr;
   bool own_shape = false;  // a launch shape was set: the bins keep their own kernels
   int *d_flag = nullptr;         // plan_match's result
@@ -164,19 +165,22 @@ hipError_t alloc_park(sgm_plan *p, const std::vector<unsigned long long> &keys) 
   if (e == hipSuccess && total > 0)
     e = hipMalloc(&p->d_rec, sizeof(double) * stride * (size_t)total);
   if (e == hipSuccess && total > 0) e = hipMalloc(&p->d_cell_of, sizeof(int) * total);
-  std::vector<int> small(5 * BATCH_SMALL, 0);
+  std::vector<BatchBin> batch(BATCH_BINS, BatchBin{});
   std::vector<long> range(14, 0);
   long first = 0;
   for (size_t bi = 0; bi < p->bins.size(); ++bi) {
     const Bin &b = p->bins[bi];
     if (b.nm < 2 || b.nm > 6) continue;
-    small[BATCH_SMALL * (b.nm - 2)] = (int)first;
-    small[BATCH_SMALL * (b.nm - 2) + 1] = (int)nrec[bi];
+    batch[b.nm - 2].first = (int)first;
+    batch[b.nm - 2].records = (int)nrec[bi];
     range[2 * (b.nm - 1)] = b.start;
     range[2 * (b.nm - 1) + 1] = b.n;
     first += nrec[bi];
   }
-  if (e == hipSuccess) e = up(&p->d_small, small);
+  if (e == hipSuccess) e = hipMalloc(&p->d_batch, sizeof(BatchBin) * batch.size());
+  if (e == hipSuccess)
+    e = hipMemcpy(p->d_batch, batch.data(), sizeof(BatchBin) * batch.size(),
+                  hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMalloc(&p->d_range, sizeof(long) * range.size());
   if (e == hipSuccess)
     e = hipMemcpy(p->d_range, range.data(), sizeof(long) * range.size(), hipMemcpyHostToDevice);
@@ -189,8 +193,8 @@ hipError_t alloc_park(sgm_plan *p, const std::vector<unsigned long long> &keys) 
     k.rec = p->d_rec + first * stride;
     k.cell_of = p->d_cell_of + first;
     first += nrec[bi];
-    k.l2_count = p->d_small + BATCH_SMALL * (b.nm - 2) + 3;
-    k.l2_next = k.l2_count + 1;
+    k.l2_count = &p->d_batch[b.nm - 2].l2_count;
+    k.l2_next = &p->d_batch[b.nm - 2].l2_next;
     k.after2 = 4;
     k.run_of = p->d_run_of + b.start;
     k.run_base = p->d_run_base + run0[bi];
@@ -210,12 +214,13 @@ void free_park(sgm_plan *p) {
     b.park.rec = nullptr;
     b.park.cell_of = nullptr;
   }
-  for (void *q : {(void *)p->d_rec, (void *)p->d_range})
+  for (void *q : {(void *)p->d_rec, (void *)p->d_batch, (void *)p->d_range})
     if (q) (void)hipFree(q);
   p->d_rec = nullptr;
+  p->d_batch = nullptr;
   p->d_range = nullptr;
   for (int **q : {&p->d_run_of, &p->d_run_base, &p->d_run_cap, &p->d_run_count, &p->d_wave_run,
-                  &p->d_wave_first, &p->d_cell_of, &p->d_small}) {
+                  &p->d_wave_first, &p->d_cell_of}) {
     if (*q) (void)hipFree(*q);
     *q = nullptr;
   }
@@ -224,16 +229,18 @@ void free_park(sgm_plan *p) {
 // Zeroes the bin counters, the straggler claim counters and the batch tables'
 // counters (with parking off too: sgm_plan_tail_counts then reports zeros). A
 // fill kernel, so the reset can be captured.
-__global__ void reset_kernel(int *counters, int nbins, int *run_count, int nruns, int *small) {
+__global__ void reset_kernel(int *counters, int nbins, int *run_count, int nruns,
+                             BatchBin *bins) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nbins) counters[i] = 0;
   if (run_count && i < nruns) run_count[i] = 0;
-  if (small && i < 5 * BATCH_SMALL && i % BATCH_SMALL >= 2) small[i] = 0;
+  if (bins && i < BATCH_BINS)
+    bins[i].claimed = bins[i].next = bins[i].l2_count = bins[i].l2_next = 0;
 }
 hipError_t reset_counters(sgm_plan *p, hipStream_t s) {
-  const int n = std::max(std::max((int)p->bins.size(), p->nruns), 5 * BATCH_SMALL);
+  const int n = std::max(std::max((int)p->bins.size(), p->nruns), BATCH_BINS);
   reset_kernel<<<(n + 255) / 256, 256, 0, s>>>(p->d_counters, (int)p->bins.size(),
-                                                p->d_run_count, p->nruns, p->d_small);
+                                                p->d_run_count, p->nruns, p->d_batch);
   return hipGetLastError();
 }
 
@@ -309,7 +316,7 @@ hipError_t launch_bins(sgm_plan *p, const PteArgs &a, const MixParamsDev &P, hip
         return e;
     }
     BatchArgs b;
-    b.small = p->d_small;
+    b.bins = p->d_batch;
     b.rec = p->d_rec;
     b.cell_of = p->d_cell_of;
     b.stride = ParkStride(p->method, BinMaxNM(p->method));
@@ -563,16 +570,16 @@ int sgm_plan_describe(const sgm_plan *p, long *out, int max_bins) {
 int sgm_plan_tail_counts(const sgm_plan *p, int *out, int max_bins, sgm_stream_t stream) {
   if (!p || !out || max_bins < 0) return SGM_E_ARG;
   const int nb = (int)p->bins.size();
-  std::vector<int> c(5 * BATCH_SMALL, 0);
-  if (p->d_small) {
+  std::vector<BatchBin> c(BATCH_BINS, BatchBin{});
+  if (p->d_batch) {
     hipStream_t s = (hipStream_t)stream;
-    if (hipMemcpyAsync(c.data(), p->d_small, sizeof(int) * c.size(), hipMemcpyDeviceToHost, s) !=
-            hipSuccess ||
+    if (hipMemcpyAsync(c.data(), p->d_batch, sizeof(BatchBin) * c.size(), hipMemcpyDeviceToHost,
+                       s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
       return SGM_E_HIP;
   }
   for (int i = 0; i < nb && i < max_bins; ++i)
-    out[i] = p->bins[i].park.rec ? c[BATCH_SMALL * (p->bins[i].nm - 2) + 3] : 0;
+    out[i] = p->bins[i].park.rec ? c[p->bins[i].nm - 2].l2_count : 0;
   return nb;
 }
 

@@ -564,22 +564,22 @@ __attribute__((amdgpu_waves_per_eu(WPE, WPE))) pte_tail_kernel(PteArgs a, MixPar
 template <int NM>
 __device__ __forceinline__ ParkArgs batch_park(const BatchArgs &b) {
   ParkArgs pk;
-  int *sm = b.small + BATCH_SMALL * (NM - 2);
+  BatchBin *t = b.bins + (NM - 2);
   pk.after = b.after;
   pk.stride = b.stride;
   pk.rec = b.rec;
   pk.cell_of = b.cell_of;
-  pk.run_base = sm;
-  pk.run_cap = sm + 1;
-  pk.run_count = sm + 2;
+  pk.run_base = &t->first;
+  pk.run_cap = &t->records;
+  pk.run_count = &t->claimed;
   // one run: its claimed records; -1 where the batch's parked cells go to the
   // team kernel
   int parked = 0;
-  for (int k = 0; k < 5; ++k) parked += b.small[BATCH_SMALL * k + 2];
+  for (int k = 0; k < BATCH_BINS; ++k) parked += b.bins[k].claimed;
   pk.nwaves = parked <= TEAM_MAX ? -1 : 0;
   pk.after2 = b.after2;
-  pk.l2_count = sm + 3;
-  pk.l2_next = sm + 4;
+  pk.l2_count = &t->l2_count;
+  pk.l2_next = &t->l2_next;
   return pk;
 }
 template <int METHOD>
@@ -595,8 +595,8 @@ pte_batch_bins_kernel(PteArgs a, MixParamsDev P, BatchArgs b, const int *__restr
 #define SGM_ONE(K)                                                                             \
   case K:                                                                                      \
     if constexpr (K <= BinMaxNM(METHOD))                                                       \
-      bin_body<K, METHOD>(lds, a, P, cells + r[0], r[1], b.small + BATCH_SMALL * (K - 2) + 5,  \
-                          chunk, batch_park<K>(b));                                            \
+      bin_body<K, METHOD>(lds, a, P, cells + r[0], r[1], &b.bins[K - 2].next, chunk,          \
+                          batch_park<K>(b));                                                   \
     break;
   switch (nm) { SGM_ONE(2) SGM_ONE(3) SGM_ONE(4) SGM_ONE(5) SGM_ONE(6) }
 #undef SGM_ONE
@@ -607,8 +607,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, LEVE
 pte_batch_tails_kernel(PteArgs a, MixParamsDev P, BatchArgs b, int resident, int wide_max) {
   extern __shared__ EosDev lds[];
   const int nm = BinMaxNM(METHOD) - (int)blockIdx.y;
-  const int *sm = b.small + BATCH_SMALL * (nm - 2);
-  if (sm[2] == 0 || (LEVEL == 2 && sm[3] == 0)) return;  // nothing parked
+  const BatchBin &t = b.bins[nm - 2];
+  if (t.claimed == 0 || (LEVEL == 2 && t.l2_count == 0)) return;  // nothing parked
   stage_registry(lds, a.d_eos, a.nreg);
 #define SGM_ONE(K)                                                                             \
   case K:                                                                                      \
@@ -693,10 +693,9 @@ __global__ void __launch_bounds__(64 * 6) pte_batch_team_kernel(PteArgs a, MixPa
                                                                 BatchArgs b) {
   extern __shared__ EosDev lds[];
   const int nm = BinMaxNM(METHOD) - (int)blockIdx.y;
-  const int *sm = b.small + BATCH_SMALL * (nm - 2);
-  const int claimed = min(sm[2], sm[1]);
+  const int claimed = min(b.bins[nm - 2].claimed, b.bins[nm - 2].records);
   int parked = 0;
-  for (int k = 0; k < 5; ++k) parked += b.small[BATCH_SMALL * k + 2];
+  for (int k = 0; k < BATCH_BINS; ++k) parked += b.bins[k].claimed;
   if (parked > TEAM_MAX || (int)blockIdx.x >= claimed) return;
   stage_registry(lds, a.d_eos, a.nreg);
 #define SGM_ONE(K)                                                                             \

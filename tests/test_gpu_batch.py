@@ -169,3 +169,69 @@ def test_pair_kernel_matches_plain_kernel(sgm, workloads, torch_gpu, method, n):
     m = mixed.result()
     assert same({k: v[3 if k in FIELDS else 1:] for k, v in m.items()}, ref)
     ctx.close()
+
+
+class PlanRun:
+    """A plan over a call's cells, executed on its working arrays."""
+
+    def __init__(self, sgm, ctx, call):
+        self.call = call
+        self.plan = sgm.Plan(ctx, call.n, call.nnz, call.off, call.mat, call.method)
+
+    def run(self):
+        c = self.call
+        for k in FIELDS:
+            c.w[k].copy_(c.base[k])
+        assert self.plan.execute(c.w["rho"], c.w["vfrac"], c.w["sie"], c.w["temp"], c.w["press"],
+                                 c.vt, c.cin, params=c.params, resid=c.resid, **c.st) == 0
+        return c
+
+    def ms(self, torch):
+        """Fastest of seven executions (without the copies) after two more."""
+        t = []
+        for _ in range(9):
+            for k in FIELDS:
+                self.call.w[k].copy_(self.call.base[k])
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            c = self.call
+            e[0].record()
+            assert self.plan.execute(c.w["rho"], c.w["vfrac"], c.w["sie"], c.w["temp"],
+                                     c.w["press"], c.vt, c.cin, params=c.params, resid=c.resid,
+                                     **c.st) == 0
+            e[1].record()
+            torch.cuda.synchronize()
+            t.append(e[0].elapsed_time(e[1]))
+        return min(t[2:])
+
+
+def pair_context(sgm, workloads):
+    ctx = sgm.Context(2)
+    ctx.set_ideal(0, *workloads.IDEAL_A)
+    ctx.set_stiff(1, *workloads.STIFF_B)
+    return ctx
+
+
+@pytest.mark.parametrize("pool,n", [("pair", 1 << 18), ("uneven", 30011)])
+def test_set_shape_changes_the_schedule_only(sgm, workloads, torch_gpu, pool, n):
+    """The shared launch of a plan's bins against a kernel per bin (a launch
+    shape set, the default one): the same bits, and over many two-material
+    cells the shared launch keeps pace (its counters once shared a cache line
+    with what every wave reads: 1.6 times the per-bin kernel's time)."""
+    torch = torch_gpu
+    if pool == "pair":
+        ctx = pair_context(sgm, workloads)
+        a = workloads.pte2(n)
+    else:
+        ctx, _ = workloads.pool_context()
+        a = workloads.uneven(ctx, n, seed=0x5EED0000 + 960)
+    p = PlanRun(sgm, ctx, Call(torch, sgm, a, 0, tight=pool == "uneven"))
+    shared = p.run().result()
+    shared_ms = p.ms(torch)
+    for i, b in enumerate(p.plan.describe()):
+        if 2 <= b["nmat"] <= 6:
+            p.plan.set_shape(i, b["block"], b["cells_per_wave"], b["grid"])
+    assert same(p.run().result(), shared)
+    if pool == "pair":
+        assert shared_ms < 1.25 * p.ms(torch)
+    p.plan.close()
+    ctx.close()
