@@ -493,6 +493,27 @@ int sgm_vec_rhoe_from_PT(sgm_ctx *ctx, int m, const double *P, const double *T, 
              : SGM_E_HIP;
 }
 
+// Whether a plain call keeps the plain kernel although its cells hold more than
+// two materials: k = nnz / ncell materials in each of them (any mix of counts
+// that averages to exactly k is taken for it), all of them gases or stiffened
+// gases, whose cells finish within a few passes of each other. Its waves then
+// run one count of materials, and neither the batch's sort nor its parking has
+// anything to save: 3 materials 435 us against 542 as a batch, 6 at fixed
+// temperature 600 against 1,176 (65,536 cells); any other mix of counts costs
+// the plain kernel the sum over them (2 to 6: 3.2 ms against 1.2). Past one
+// wave of cells per SIMD the plain kernel takes a second round: 131,072 cells of
+// 3 materials 781 us against 635, but at fixed temperature 352 against 470, and
+// 262,144 of 6 materials 3.7 ms against 4.0.
+static bool uniform_gases(const sgm_ctx *ctx, int method, long ncell, long nnz) {
+  if (nnz % ncell != 0) return false;
+  if (ncell > 256L * device_cu_count() && nnz / ncell <= 4 && method != PTE_FIXED_T) return false;
+  for (int i = 0; i < ctx->nmat; ++i)
+    if (ctx->is_set[i] && ctx->host_eos[i].kind != KIND_IDEAL &&
+        ctx->host_eos[i].kind != KIND_STIFF)
+      return false;
+  return true;
+}
+
 static int pte_common(int method, sgm_ctx *ctx, long ncell, long nnz, const int *offsets,
                       const uint8_t *mat_ids, double *rho, double *vfrac, double *sie,
                       double *temp, double *press, const double *vfrac_tot,
@@ -531,14 +552,15 @@ static int pte_common(int method, sgm_ctx *ctx, long ncell, long nnz, const int 
   const MixParamsDev P = to_dev(params);
   // More than two materials per cell on average: the batched kernels (a
   // sort and some twenty launches, about 0.15 ms, against the plain kernel's
-  // lanes held by their waves' slowest cells: 7 to 20 times the time on
-  // uneven cells of 100 to 20,000). Two-material cells finish within a few
-  // passes of each other. RhoU has no bins past four materials and cells with
+  // lanes held by their waves' slowest cells: the same time at one uneven
+  // cell, 2 to 20 times less from 4 to 20,000; 65,536 pairs and one cell of
+  // three 388 us against 447, 500,000 and one 1,234 against 1,335).
+  // Two-material cells finish within a few passes of each other. RhoU has no bins past four materials and cells with
   // modified materials none at all: their list kernel would run behind the
   // other cells' tails instead of beside them (RhoU, 1,000 uneven cells: 265 ms
   // plain, 310 to 350 as a batch).
   const bool binned = method != PTE_RHOU && ctx_mod_mask(ctx) == 0;
-  if (nnz > 2 * ncell && binned) {
+  if (nnz > 2 * ncell && binned && !uniform_gases(ctx, method, ncell, nnz)) {
     bool taken = false;
     const hipError_t e = launch_pte_batch(ctx, method, a, P, (hipStream_t)stream, taken);
     if (e != hipSuccess) return SGM_E_HIP;

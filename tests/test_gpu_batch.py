@@ -235,3 +235,57 @@ def test_set_shape_changes_the_schedule_only(sgm, workloads, torch_gpu, pool, n)
         assert shared_ms < 1.25 * p.ms(torch)
     p.plan.close()
     ctx.close()
+
+
+def replay_ms(torch, ctx, call):
+    """Fastest of seven replays of the call's plain kernels (captured)."""
+    g = torch.cuda.CUDAGraph()
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s), torch.cuda.graph(g, stream=s):
+        call.run(ctx, s.cuda_stream)
+    t = []
+    for _ in range(9):
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        e[0].record()
+        g.replay()
+        e[1].record()
+        torch.cuda.synchronize()
+        t.append(e[0].elapsed_time(e[1]))
+    return min(t[2:]), call.result()
+
+
+def call_ms(torch, ctx, call):
+    t = []
+    for _ in range(9):
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        e[0].record()
+        call.run(ctx, 0)
+        e[1].record()
+        torch.cuda.synchronize()
+        t.append(e[0].elapsed_time(e[1]))
+    return min(t[2:]), call.result()
+
+
+@pytest.mark.parametrize("method,k,n", [(0, 3, 65536), (2, 6, 65536), (1, 3, 16384),
+                                        (2, 4, 140000)])
+def test_uniform_gas_calls_keep_pace_with_the_plain_kernel(sgm, workloads, torch_gpu, method, k,
+                                                           n):
+    """k materials, gases and a stiffened gas, in every cell: the call against
+    its plain kernels (as a batch it took 1.2 to 1.95 times as long)."""
+    torch = torch_gpu
+    ctx = pair_context(sgm, workloads)
+    p = workloads.pte2(n, seed=0x5EED0000 + 970)
+    a = dict(p, ncell=n, nnz=k * n, offsets=np.arange(0, k * n + 1, k, dtype=np.int32))
+    split = np.ones(k)  # the gas of each pair split over k - 1 entries
+    split[:k - 1] = 1.0 / (k - 1)
+    src = np.array([0] * (k - 1) + [1])
+    for f in FIELDS:
+        v = p[f].reshape(n, 2)[:, src]
+        a[f] = (v * split if f == "vfrac" else v).ravel().copy()
+    a["mat_ids"] = np.tile(src.astype(np.uint8), n)
+    call = Call(torch, sgm, a, method, tight=False)
+    got_ms, got = call_ms(torch, ctx, call)
+    plain_ms, plain = replay_ms(torch, ctx, call)
+    assert same(got, plain)
+    assert got_ms < 1.15 * plain_ms + 0.03
+    ctx.close()
