@@ -15,12 +15,12 @@
 #include <algorithm>
 
 namespace sgm {
-// Lanes of a wave that take cells: all 64 once the batch fills four waves per
-// CU with them, fewer below, where waves are plentiful and each pass of a
-// wave costs the sum of its lanes' material kinds.
-int batch_cells_per_wave(long ncell, int ncu) {
+// Lanes of a wave that take cells: all 64 once the cells fill `waves` waves
+// with them, fewer below, where waves are plentiful and each pass of a wave
+// costs the sum of its lanes' material kinds.
+int batch_cells_per_wave(long ncell, long waves) {
   int c = 64;
-  while (c > 4 && ncell < 4L * ncu * c) c /= 2;
+  while (c > 4 && ncell < waves * c) c /= 2;
   return c;
 }
 
@@ -123,7 +123,7 @@ hipError_t enqueue(int method, const PteArgs &a, const MixParamsDev &P,
   b.after = BATCH_PARK_AFTER;
   b.after2 = BATCH_AFTER2;
   e = launch_pte_batch_bins(method, a, P, b, sorted, range, n,
-                            batch_cells_per_wave(n, device_cu_count()), s);
+                            batch_cells_per_wave(n, 4L * device_cu_count()), s);
   for (int side = 0; side < 2 && e == hipSuccess; ++side)
     e = launch_pte_list(method, a, P, sorted, n, s, range + (side ? 2 * (NBIN + 1) : 0));
   return e;

@@ -99,7 +99,7 @@ inline unsigned long long ctx_mod_mask(const sgm_ctx *ctx) {
 // captured, or there is no memory for the work arrays).
 hipError_t launch_pte_batch(sgm_ctx *ctx, int method, const PteArgs &a, const MixParamsDev &P,
                             hipStream_t s, bool &taken);
-int batch_cells_per_wave(long ncell, int ncu);
+int batch_cells_per_wave(long ncell, long waves);
 // the batch itself, its work arrays in buf (batch_bytes); nrec: straggler
 // records per material count, 0: one per cell
 size_t batch_bytes(int method, long n, int nrec);

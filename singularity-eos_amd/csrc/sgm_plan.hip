@@ -286,12 +286,32 @@ std::vector<size_t> bin_order(const sgm_plan *p) {
   return order;
 }
 
-// A plan launches its bins together (one kernel for all bins, one per tail
-// level: launch_pte_batch_bins) unless a launch shape was set for one, or for
-// RhoU, whose cells past four materials have no bin: the bins then keep their
-// own kernels, each bin's tail beside the next bins'.
-// Together against apart: 2^17 cells of get_sg_eos 63 -> 55 ms, plans of 2,517
-// cells 10.2 -> 4.7 ms, 142,921 14.6 -> 13.1, 2^19 17.5 -> 15.3, 2^20 21.9 -> 19.0.
+// Whether a plan launches its bins together (one kernel for all bins, one per
+// tail level: launch_pte_batch_bins): unless a launch shape was set for one,
+// and not for RhoU, whose cells past four materials have no bin. The bins then
+// keep their own kernels, each bin's tail beside the next bins'. Apart against
+// together, uneven cells: RhoT 1,000 8.3 / 1.9 ms, 2^16 11.5 / 7.8, 2^20 21.3 /
+// 17.2; FixedT 2^14 4.9 / 3.6, 2^20 15.6 / 14.0. The shared tails take the
+// parked cells in claim order, the bins' own by signature: where the parked
+// cells outnumber the chip's waves and each pass is long, a wave of one
+// signature is the faster. PT 1,000 175 / 75 ms, 2^14 250 / 194, 2^15 246 / 211,
+// 2^16 249 / 261, 2^17 235 / 329; FixedP 2^16 46.7 / 37.3, 2^18 97 / 83,
+// 2^20 156 / 165.
+bool shared_launch(const sgm_plan *p) {
+  const long most = p->method == PTE_PT        ? 1L << 15
+                    : p->method == PTE_FIXED_P ? 1L << 19
+                                               : 1L << 31;
+  return !p->own_shape && p->d_rec && p->method != PTE_RHOU && p->ncell <= most;
+}
+// Lanes of a wave that take cells: the cells of a plan spread over four waves
+// per CU; over one where each bin holds one signature, whose lanes run the same
+// material kinds in any case, so that more waves only compete for the
+// instruction cache (4,096 two-material cells 229 -> 198 us, 16,384 221 -> 194).
+int plan_cells_per_wave(const sgm_plan *p) {
+  int bins = 0;
+  for (const Bin &b : p->bins) bins += b.nruns > 0;
+  return batch_cells_per_wave(p->ncell, (p->nruns == bins ? 1L : 4L) * device_cu_count());
+}
 
 // Records the counter reset and every bin on stream s: the persistent bin
 // kernels one after another on s; with fork streams (graph capture, or a
@@ -302,7 +322,7 @@ hipError_t launch_bins(sgm_plan *p, const PteArgs &a, const MixParamsDev &P, hip
                        bool fork) {
   hipError_t e = reset_counters(p, s);
   if (e != hipSuccess) return e;
-  if (!p->own_shape && p->d_rec && p->method != PTE_RHOU) {
+  if (shared_launch(p)) {
     // the list bins beside the batch, each on a stream of its own
     const bool lists = fork && p->aux.size() >= p->bins.size() &&
                        p->ev.size() >= 2 * p->bins.size();
@@ -323,7 +343,7 @@ hipError_t launch_bins(sgm_plan *p, const PteArgs &a, const MixParamsDev &P, hip
     b.after = p->park_after;
     b.after2 = 4;
     e = launch_pte_batch_bins(p->method, a, P, b, p->d_sorted, p->d_range, p->ncell,
-                              batch_cells_per_wave(p->ncell, device_cu_count()), s);
+                              plan_cells_per_wave(p), s);
     for (size_t i = 0; i < p->bins.size() && e == hipSuccess; ++i) {
       const Bin &x = p->bins[i];
       if (x.nm >= 2 && x.nm <= 6) continue;
