@@ -320,6 +320,7 @@ int plan_cells_per_wave(const sgm_plan *p) {
 // tails run beside the later bins. Without forks everything stays on s.
 hipError_t launch_bins(sgm_plan *p, const PteArgs &a, const MixParamsDev &P, hipStream_t s,
                        bool fork) {
+  if (p->bins.empty()) return hipSuccess;  // get_sg_eos without a mixed cell
   hipError_t e = reset_counters(p, s);
   if (e != hipSuccess) return e;
   if (shared_launch(p)) {
