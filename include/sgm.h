@@ -339,17 +339,20 @@ int sgm_driver_cache_info(sgm_ctx *ctx, long *out);
 /* ---- PTE closure (batched, persistent, hipGraph path) -------------------- */
 /* No reference counterpart: a plan bins the cells of a fixed CSR topology by
  * material count (2..6 run register-resident templated kernels; 2..4 for
- * RhoU; 9..64 one wave per cell) and by material signature, autotunes block
- * shape and cells-per-wave
- * per bin, and captures one hipGraph whose persistent kernel nodes solve
- * every bin. method: 0 = RhoT, 1 = PT, 2 = FixedT, 3 = FixedP (the per-cell
+ * RhoU; 9..64 one wave per cell) and by material signature and captures one
+ * hipGraph whose persistent kernel nodes solve every bin: one node for all
+ * register-resident bins, or one per bin (RhoU, large PT and FixedP plans, and
+ * after sgm_plan_set_shape or an autotuning that found it faster). method: 0 = RhoT, 1 = PT, 2 = FixedT, 3 = FixedP (the per-cell
  * sie_tot array of execute then holds the cell temperature / pressure, and
  * Tnorm is ignored), 4 = RhoU. Results are identical to sgm_pte_rhoT /
  * sgm_pte_PT / sgm_pte_fixedT / sgm_pte_fixedP / sgm_pte_rhoU on the same
  * inputs. The plan keeps device copies of offsets and mat_ids. */
 int sgm_plan_create(sgm_ctx *ctx, long ncell, long nnz, const int *offsets,
                     const uint8_t *mat_ids, int method, sgm_plan **plan, sgm_stream_t stream);
-/* autotune (optional; uses the given arrays as scratch-copied input) */
+/* autotune (optional; uses the given arrays as scratch-copied input): times
+ * launch shapes per bin, then whole executions of a kernel per bin in the
+ * fastest shapes against the plan's schedule so far, and keeps the faster. On
+ * an error the plan keeps the schedule it had. Results do not change. */
 int sgm_plan_autotune(sgm_plan *plan, const double *rho, const double *vfrac,
                       const double *temp, const double *press, const double *vfrac_tot,
                       const double *sie_tot, const sgm_mix_params *params, int reps,
@@ -360,7 +363,8 @@ int sgm_plan_execute(sgm_plan *plan, double *rho, double *vfrac, double *sie, do
                      sgm_pte_status status, sgm_stream_t stream);
 /* No reference counterpart: sets one register-resident bin's launch shape
  * (block 64/128/256 threads, cells claimed per wave >= 64, persistent grid),
- * as sgm_plan_autotune would. Results do not change. */
+ * and with it a kernel per bin for every bin of the plan. Results do not
+ * change. */
 int sgm_plan_set_shape(sgm_plan *plan, int bin, int block, int cells_per_wave, int grid);
 /* No reference counterpart. Cells of the register-resident bins that are
  * still iterating after `iterations` Newton iterations are parked (their

@@ -239,6 +239,25 @@ def test_default_schedule_keeps_pace(sgm, workloads, torch_gpu, pool, method, n,
     ctx.close()
 
 
+@pytest.mark.parametrize("n", [2517, 40000])
+def test_autotune_keeps_the_faster_schedule(sgm, workloads, torch_gpu, n):
+    """Autotuning picks shapes for a kernel per bin; the plan takes them only
+    where whole executions are faster than its own schedule (it once always
+    did: 2,517 cells 4.2 -> 13.2 ms). Same bits either way."""
+    torch = torch_gpu
+    ctx, _ = workloads.pool_context()
+    call = Call(torch, sgm, workloads.uneven(ctx, n, seed=0x5EED0000 + 980), 0, True)
+    p = PlanRun(sgm, ctx, call)
+    before, want = p.ms(torch), call.result()
+    b = call.base
+    p.plan.autotune(b["rho"], b["vfrac"], b["temp"], b["press"], call.vt, call.cin,
+                    params=call.params, reps=1)
+    assert p.ms(torch) < 1.2 * before
+    assert same(call.result(), want)
+    p.plan.close()
+    ctx.close()
+
+
 def replay_ms(torch, ctx, call):
     """Fastest of seven replays of the call's plain kernels (captured)."""
     g = torch.cuda.CUDAGraph()
