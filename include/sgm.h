@@ -200,8 +200,9 @@ int sgm_vec_rhoe_from_PT(sgm_ctx *ctx, int matindex, const double *P, const doub
  * Calls with more than two materials per cell on average (no material with
  * modifiers; not sgm_pte_rhoU) sort their cells on the device first, in work
  * arrays the context keeps between calls (about 0.8 KB per cell of the
- * largest call, at most 2^20 cells' worth and at most four sets, for calls
- * that overlap on several streams; sgm_finalize frees them). While the stream
+ * largest call, up to a quarter more once it has grown, at most 2^20 cells'
+ * worth and at most four sets, for calls that overlap on several streams;
+ * sgm_release_driver_cache and sgm_finalize free them). While the stream
  * is being captured, or when there is no memory for them, the call runs on
  * kernels that need none. The results are the same. */
 int sgm_pte_rhoT(sgm_ctx *ctx, long ncell, long nnz, const int *offsets, const uint8_t *mat_ids,
@@ -327,8 +328,8 @@ int sgm_get_sg_eos_noalloc(sgm_ctx *ctx, int nmat, int ncell, int cell_dim, int 
                            sgm_stream_t stream);
 /* No reference counterpart: frees the work buffers and the batched plan that
  * sgm_get_sg_eos keeps in the context between calls (for the 2^20-cell
- * uneven workload about 0.8 GB of straggler records plus the arenas); the
- * next call rebuilds them. This memory is outside any server's
+ * uneven workload about 0.8 GB of straggler records plus the arenas), and the
+ * work arrays of plain closure calls; the next calls rebuild them. This memory is outside any server's
  * hbm_budget_bytes. sgm_finalize releases it too. */
 int sgm_release_driver_cache(sgm_ctx *ctx);
 /* No reference counterpart: out[4] (HOST) = {calls that built the driver's

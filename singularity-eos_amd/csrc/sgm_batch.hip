@@ -196,16 +196,26 @@ hipError_t launch_pte_batch(sgm_ctx *ctx, int method, const PteArgs &a, const Mi
     return hipSuccess;
   }
   if (ws->bytes < L.total) {
+    // growing waits for the last call and for the device (hipFree): a quarter
+    // of headroom, so that calls whose cells creep up pay it now and then
+    // instead of at every new largest call (79 us of host time against 50, and
+    // whatever else the device had in flight)
+    const size_t more = std::min(ws->bytes + ws->bytes / 4,
+                                 batch_bytes(method, BATCH_MAX_CELLS, 0));
     if (hipEventSynchronize(ws->done) != hipSuccess) return hipSuccess;
     if (ws->buf) (void)hipFree(ws->buf);
     ws->buf = nullptr;
+    const size_t sizes[2] = {ws->bytes ? std::max(L.total, more) : L.total, L.total};
     ws->bytes = 0;
-    if (hipMalloc(&ws->buf, L.total) != hipSuccess) {
+    for (size_t want : sizes) {
+      if (hipMalloc(&ws->buf, want) == hipSuccess) {
+        ws->bytes = want;
+        break;
+      }
       (void)hipGetLastError();
       ws->buf = nullptr;
-      return hipSuccess;  // no room: the plain kernel needs none
     }
-    ws->bytes = L.total;
+    if (!ws->buf) return hipSuccess;  // no room: the plain kernel needs none
   } else if (hipStreamWaitEvent(s, ws->done, 0) != hipSuccess) {
     return hipErrorUnknown;
   }

@@ -238,7 +238,6 @@ int sgm_finalize(sgm_ctx *ctx) {
   }
   hipDeviceSynchronize();
   sgm_release_driver_cache(ctx);
-  for (auto &w : ctx->batch) w.release();
   for (auto &t : ctx->tables)
     if (t)
       for (void *p : t->d_arrays) hipFree(p);
@@ -251,6 +250,10 @@ int sgm_finalize(sgm_ctx *ctx) {
 
 int sgm_release_driver_cache(sgm_ctx *ctx) {
   if (!ctx) return SGM_E_ARG;
+  {
+    std::lock_guard<std::mutex> g(ctx->batch_mu);
+    for (auto &w : ctx->batch) w.release();
+  }
   std::lock_guard<std::mutex> g(ctx->drv_mu);
   if (ctx->drv_plan) sgm_plan_destroy(ctx->drv_plan);
   if (ctx->drv_cells) (void)hipFree(ctx->drv_cells);

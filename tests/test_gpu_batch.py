@@ -310,3 +310,30 @@ def test_uniform_gas_calls_keep_pace_with_the_plain_kernel(sgm, workloads, torch
     assert same(got, plain)
     assert got_ms < 1.15 * plain_ms + 0.03
     ctx.close()
+
+
+def test_work_arrays_grow_with_headroom_and_are_given_back(sgm, workloads, torch_gpu):
+    """Calls of slowly rising size allocate now and then, not each time (every
+    allocation frees the last one, which waits for the whole device), and
+    sgm_release_driver_cache gives the memory back."""
+    torch = torch_gpu
+    ctx, _ = workloads.pool_context()
+    sizes = range(30000, 90000, 3000)
+    a = workloads.uneven(ctx, sizes[-1], seed=0x5EED0000 + 990)
+    call = Call(torch, sgm, a, 2, tight=False)
+    off = a["offsets"]
+    torch.cuda.synchronize()
+    free = [torch.cuda.mem_get_info()[0]]
+    for n in sizes:
+        call.n, call.nnz = n, int(off[n])
+        call.run(ctx, 0)
+        torch.cuda.synchronize()
+        free.append(torch.cuda.mem_get_info()[0])
+    assert sum(x != y for x, y in zip(free, free[1:])) <= 7  # 1.25^6 = 3.8
+    held = free[0] - free[-1]
+    assert held > 0.5e3 * sizes[-1]
+    assert sgm.lib().sgm_release_driver_cache(ctx.h) == 0
+    assert torch.cuda.mem_get_info()[0] - free[-1] >= held - (4 << 20)
+    call.run(ctx, 0)  # and the next call allocates again
+    torch.cuda.synchronize()
+    ctx.close()
