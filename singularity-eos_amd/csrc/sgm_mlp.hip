@@ -107,6 +107,14 @@ __device__ __forceinline__ void w_store(const u4 (&r)[N], bf16 *dst, int ld) {
     *reinterpret_cast<u4 *>(dst + (c / (COLS / 8)) * ld + (c % (COLS / 8)) * 8) = r[i];
   }
 }
+// LDS written by some lanes of a wave before it, read by others after it. The
+// barrier alone orders no memory for the compiler; the fences do, and cost no
+// instruction (a wave's LDS operations execute in order).
+__device__ __forceinline__ void wave_handover() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 // 16 features of a row: two 16-byte loads, or, where the caller's matrix is not
 // on a 16-byte boundary, one by one
 __device__ __forceinline__ void load_features(const bf16 *p, bool aligned, u4 (&x)[2]) {
@@ -187,18 +195,18 @@ __device__ __forceinline__ void infer_rows(InferLds &L, const float *__restrict_
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   bf16 *row = L.row + w * 16 * LDH;
   hidden_layer<false>(row, L.w1, LDK, KIN, P + OB1, nullptr, 0, nullptr);
-  __builtin_amdgcn_wave_barrier();
+  wave_handover();
   hidden_layer<false>(row, L.w2, LDH, H, P + OB2, nullptr, 0, nullptr);
-  __builtin_amdgcn_wave_barrier();
+  wave_handover();
   hidden_layer<false>(row, L.w3, LDH, H, P + OB3, nullptr, 0, nullptr);
-  __builtin_amdgcn_wave_barrier();
+  wave_handover();
   f4 acc[1] = {f4{0, 0, 0, 0}};
   wave_gemm<1>(row, LDH, L.w4, LDH, H, acc);
   const float b = P[OB4 + (l & 15)];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     L.y[(w * 16 + (l >> 4) * 4 + i) * (KOUT + 1) + (l & 15)] = acc[0][i] + b;
-  __builtin_amdgcn_wave_barrier();
+  wave_handover();
 }
 
 // outputs of rows idx[0..B) of the feature matrix Xall [N][KIN]
@@ -218,13 +226,13 @@ __global__ void __launch_bounds__(512, 1) fwd_kernel(const bf16 *__restrict__ wq
     u4 *d = reinterpret_cast<u4 *>(L.row + (w * 16 + (l >> 2)) * LDH + (l & 3) * 16);
     d[0] = x[0];
     d[1] = x[1];
-    __builtin_amdgcn_wave_barrier();
+    wave_handover();
     infer_rows(L, P);
     for (int k = l; k < 16 * KOUT; k += 64) {
       const long rr = t * 16 + k / KOUT;
       if (rr < B) Y[rr * KOUT + k % KOUT] = L.y[(w * 16 + k / KOUT) * (KOUT + 1) + k % KOUT];
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_handover();
   }
 }
 
@@ -604,7 +612,7 @@ __global__ void __launch_bounds__(512, 1)
     for (int k = l; k < 16 * (KIN / 8); k += 64)
       *reinterpret_cast<u4 *>(row + (k / (KIN / 8)) * LDH + (k % (KIN / 8)) * 8) =
           u4{0, 0, 0, 0};
-    __builtin_amdgcn_wave_barrier();
+    wave_handover();
     if (l < 16) {
       const long c = t * 16 + l;
       int nm = 0;
@@ -630,7 +638,7 @@ __global__ void __launch_bounds__(512, 1)
       }
       L.nm[w * 16 + l] = nm;
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_handover();
     for (int k = l; k < 16 * SLOTS; k += 64) {
       const int q = k / SLOTS, s = k % SLOTS;
       if (s >= L.nm[w * 16 + q]) continue;
@@ -643,7 +651,7 @@ __global__ void __launch_bounds__(512, 1)
       x[7] = f2bf(((float)log(a.rho[e]) - mu[f + 7]) / sg[f + 7]);
       x[8] = f2bf(((float)log(a.temp[e]) - mu[f + 8]) / sg[f + 8]);
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_handover();
     infer_rows(L, P);
     if (l < 16 && t * 16 + l < a.ncell) {
       const long c = t * 16 + l;
@@ -668,7 +676,7 @@ __global__ void __launch_bounds__(512, 1)
         gT[c] = exp((double)(t_mu + t_sg * y[6]));
       }
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_handover();
   }
 }
 
