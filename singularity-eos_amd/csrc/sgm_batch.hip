@@ -34,10 +34,10 @@ constexpr int BATCH_PARK_AFTER = 20, BATCH_AFTER2 = 4;  // as plans
 // each of its cells at the cells' own positions); range 0 the cells before them (fewer than 2 materials),
 // range 6 those past the register-resident counts.
 __global__ void batch_tables_kernel(const unsigned long long *__restrict__ keys, long n,
-                                    int max_nm, int nrec, long *__restrict__ range,
+                                    int method, int nrec, long *__restrict__ range,
                                     BatchBin *__restrict__ bins) {
   __shared__ long pos[NBIN + 1];  // first position with a count of at least k + 2
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, max_nm = BinMaxNM(method);
   if (t <= NBIN) {
     const unsigned long long k = (unsigned long long)min(t + 2, max_nm + 1) << 56;
     long lo = 0, hi = n;
@@ -57,6 +57,12 @@ __global__ void batch_tables_kernel(const unsigned long long *__restrict__ keys,
     range[2 * (t + 1) + 1] = count;
     bins[t].first = nrec ? t * nrec : (int)start;
     bins[t].records = nrec ? nrec : (int)count;
+    long word = 0;
+    if (nrec)
+      for (int k = 0; k < t; ++k) word += (long)nrec * ParkStride(method, k + 2);
+    else
+      word = start * ParkStride(method, max_nm);
+    bins[t].word = word;
     bins[t].claimed = bins[t].next = bins[t].l2_count = bins[t].l2_next = 0;
   } else if (t == NBIN) {
     range[0] = 0;
@@ -85,7 +91,11 @@ hipError_t layout(int method, long n, int nrec, Layout &L) {
   L.bins = take(sizeof(BatchBin) * NBIN);
   const size_t recs = nrec ? (size_t)NBIN * nrec : (size_t)n;
   L.cell_of = take(4 * recs);
-  L.rec = take(8 * (size_t)ParkStride(method, BinMaxNM(method)) * recs);
+  size_t words = 0;  // one record per cell: a bin's start at its cells' positions
+  for (int nm = 2; nm <= BinMaxNM(method); ++nm)
+    words = nrec ? words + (size_t)ParkStride(method, nm) * nrec
+                 : (size_t)ParkStride(method, nm) * n;
+  L.rec = take(8 * words);
   size_t b = 0;
   const hipError_t e = hipcub::DeviceRadixSort::SortPairs(
       nullptr, b, (unsigned long long *)nullptr, (unsigned long long *)nullptr, (int *)nullptr,
@@ -106,20 +116,18 @@ hipError_t enqueue(int method, const PteArgs &a, const MixParamsDev &P,
   long *range = (long *)(base + L.range);
   auto *bins = (BatchBin *)(base + L.bins);
   const int n = (int)a.ncell;
-  const int max_nm = BinMaxNM(method);
   hipError_t e =
       launch_plan_keys(a.offsets, a.mat_ids, n, a.nnz, keys, ids, s, nullptr, 0, mod_mask);
   if (e != hipSuccess) return e;
   size_t tb = L.tmp_bytes;
   e = hipcub::DeviceRadixSort::SortPairs(base + L.tmp, tb, keys, keys2, ids, sorted, n, 0, 64, s);
   if (e != hipSuccess) return e;
-  batch_tables_kernel<<<1, 64, 0, s>>>(keys2, n, max_nm, nrec, range, bins);
+  batch_tables_kernel<<<1, 64, 0, s>>>(keys2, n, method, nrec, range, bins);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   BatchArgs b;
   b.bins = bins;
   b.rec = (double *)(base + L.rec);
   b.cell_of = (int *)(base + L.cell_of);
-  b.stride = ParkStride(method, max_nm);
   b.after = BATCH_PARK_AFTER;
   b.after2 = BATCH_AFTER2;
   e = launch_pte_batch_bins(method, a, P, b, sorted, range, n,

@@ -78,6 +78,7 @@ constexpr int BATCH_BINS = 5;
 struct BatchBin {
   int first;                  // the bin's first record
   int records;                // its records
+  long word;                  // where they start: FP64 words from BatchArgs::rec
   alignas(128) int claimed;   // records claimed (claims past `records` are not parked)
   alignas(128) int next;      // the cell counter
   alignas(128) int l2_count;  // as ParkArgs
@@ -86,9 +87,9 @@ struct BatchBin {
 static_assert(sizeof(BatchBin) == 512, "one line per counter");
 struct BatchArgs {
   BatchBin *bins = nullptr;
+  int min_nm = 2, max_nm = BATCH_BINS + 1;  // the material counts there may be
   double *rec = nullptr;
   int *cell_of = nullptr;
-  int stride = 0;           // FP64 words per record, every material count alike
   int after = 0, after2 = 0;  // as ParkArgs
 };
 

@@ -50,7 +50,7 @@ struct sgm_plan {
   int *d_run_of = nullptr, *d_run_base = nullptr, *d_run_cap = nullptr;
   int *d_run_count = nullptr, *d_wave_run = nullptr, *d_wave_first = nullptr;
   int nruns = 0;
-  // straggler records of all bins (one stride), and the tables of a launch
+  // straggler records of all bins, and the tables of a launch
   // whose bins share one kernel (BatchArgs): per material count its first
   // record, records, and the counters of the last execution
   double *d_rec = nullptr;
@@ -159,18 +159,21 @@ hipError_t alloc_park(sgm_plan *p, const std::vector<unsigned long long> &keys) 
   if (e == hipSuccess) e = up(&p->d_run_count, run_cap);  // contents reset per execution
   if (e == hipSuccess) e = up(&p->d_wave_run, wave_run);
   if (e == hipSuccess) e = up(&p->d_wave_first, wave_first);
-  long total = 0;
-  for (long n : nrec) total += n;
-  const int stride = ParkStride(p->method, BinMaxNM(p->method));
-  if (e == hipSuccess && total > 0)
-    e = hipMalloc(&p->d_rec, sizeof(double) * stride * (size_t)total);
+  long total = 0, words = 0;
+  for (size_t bi = 0; bi < p->bins.size(); ++bi) {
+    total += nrec[bi];
+    if (nrec[bi]) words += nrec[bi] * ParkStride(p->method, p->bins[bi].nm);
+  }
+  if (e == hipSuccess && total > 0) e = hipMalloc(&p->d_rec, sizeof(double) * (size_t)words);
   if (e == hipSuccess && total > 0) e = hipMalloc(&p->d_cell_of, sizeof(int) * total);
   std::vector<BatchBin> batch(BATCH_BINS, BatchBin{});
   std::vector<long> range(14, 0);
-  long first = 0;
+  long first = 0, word = 0;
   for (size_t bi = 0; bi < p->bins.size(); ++bi) {
     const Bin &b = p->bins[bi];
     if (b.nm < 2 || b.nm > 6) continue;
+    batch[b.nm - 2].word = word;
+    word += nrec[bi] * ParkStride(p->method, b.nm);
     batch[b.nm - 2].first = (int)first;
     batch[b.nm - 2].records = (int)nrec[bi];
     range[2 * (b.nm - 1)] = b.start;
@@ -184,13 +187,14 @@ hipError_t alloc_park(sgm_plan *p, const std::vector<unsigned long long> &keys) 
   if (e == hipSuccess) e = hipMalloc(&p->d_range, sizeof(long) * range.size());
   if (e == hipSuccess)
     e = hipMemcpy(p->d_range, range.data(), sizeof(long) * range.size(), hipMemcpyHostToDevice);
-  first = 0;
+  first = word = 0;
   for (size_t bi = 0; bi < p->bins.size() && e == hipSuccess; ++bi) {
     Bin &b = p->bins[bi];
     if (b.nm < 2 || b.nm > 6 || nrec[bi] == 0) continue;
     ParkArgs &k = b.park;
-    k.stride = stride;
-    k.rec = p->d_rec + first * stride;
+    k.stride = ParkStride(p->method, b.nm);
+    k.rec = p->d_rec + word;
+    word += nrec[bi] * k.stride;
     k.cell_of = p->d_cell_of + first;
     first += nrec[bi];
     k.l2_count = &p->d_batch[b.nm - 2].l2_count;
@@ -340,7 +344,13 @@ hipError_t launch_bins(sgm_plan *p, const PteArgs &a, const MixParamsDev &P, hip
     b.bins = p->d_batch;
     b.rec = p->d_rec;
     b.cell_of = p->d_cell_of;
-    b.stride = ParkStride(p->method, BinMaxNM(p->method));
+    b.min_nm = BinMaxNM(p->method);
+    b.max_nm = 2;
+    for (const Bin &x : p->bins) {
+      if (x.nm < 2 || x.nm > 6) continue;
+      b.min_nm = std::min(b.min_nm, x.nm);
+      b.max_nm = std::max(b.max_nm, x.nm);
+    }
     b.after = p->park_after;
     b.after2 = 4;
     e = launch_pte_batch_bins(p->method, a, P, b, p->d_sorted, p->d_range, p->ncell,

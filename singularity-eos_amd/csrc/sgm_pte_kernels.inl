@@ -561,13 +561,14 @@ __attribute__((amdgpu_waves_per_eu(WPE, WPE))) pte_tail_kernel(PteArgs a, MixPar
 // has four hardware queues: the fifth bin, and any other batch in flight,
 // would wait behind a queue's tails. The bins' kernels need the same
 // registers one by one as together.
-template <int NM>
+template <int METHOD, int NM>
 __device__ __forceinline__ ParkArgs batch_park(const BatchArgs &b) {
+  constexpr int stride = ParkStride(METHOD, NM);
   ParkArgs pk;
   BatchBin *t = b.bins + (NM - 2);
   pk.after = b.after;
-  pk.stride = b.stride;
-  pk.rec = b.rec;
+  pk.stride = stride;
+  pk.rec = b.rec + (t->word - (long)t->first * stride);
   pk.cell_of = b.cell_of;
   pk.run_base = &t->first;
   pk.run_cap = &t->records;
@@ -588,7 +589,7 @@ __attribute__((amdgpu_waves_per_eu(SGM_BIN_WAVES_PER_EU, SGM_BIN_WAVES_PER_EU)))
 pte_batch_bins_kernel(PteArgs a, MixParamsDev P, BatchArgs b, const int *__restrict__ cells,
                       const long *__restrict__ range, int chunk) {
   extern __shared__ EosDev lds[];
-  const int nm = BinMaxNM(METHOD) - (int)blockIdx.y;
+  const int nm = b.max_nm - (int)blockIdx.y;
   const long *r = range + 2 * (nm - 1);
   if ((long)blockIdx.x * chunk >= r[1]) return;  // more waves than the bin's cells fill
   stage_registry(lds, a.d_eos, a.nreg);
@@ -596,7 +597,7 @@ pte_batch_bins_kernel(PteArgs a, MixParamsDev P, BatchArgs b, const int *__restr
   case K:                                                                                      \
     if constexpr (K <= BinMaxNM(METHOD))                                                       \
       bin_body<K, METHOD>(lds, a, P, cells + r[0], r[1], &b.bins[K - 2].next, chunk,          \
-                          batch_park<K>(b));                                                   \
+                          batch_park<METHOD, K>(b));                                                   \
     break;
   switch (nm) { SGM_ONE(2) SGM_ONE(3) SGM_ONE(4) SGM_ONE(5) SGM_ONE(6) }
 #undef SGM_ONE
@@ -606,14 +607,14 @@ template <int METHOD, int LEVEL>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, LEVEL == 1 ? 2 : 1)))
 pte_batch_tails_kernel(PteArgs a, MixParamsDev P, BatchArgs b, int resident, int wide_max) {
   extern __shared__ EosDev lds[];
-  const int nm = BinMaxNM(METHOD) - (int)blockIdx.y;
+  const int nm = b.max_nm - (int)blockIdx.y;
   const BatchBin &t = b.bins[nm - 2];
   if (t.claimed == 0 || (LEVEL == 2 && t.l2_count == 0)) return;  // nothing parked
   stage_registry(lds, a.d_eos, a.nreg);
 #define SGM_ONE(K)                                                                             \
   case K:                                                                                      \
     if constexpr (K <= BinMaxNM(METHOD)) {                                                     \
-      const ParkArgs pk = batch_park<K>(b);                                                    \
+      const ParkArgs pk = batch_park<METHOD, K>(b);                                                    \
       if constexpr (LEVEL == 2 && TailWide(METHOD, K)) {                                       \
         if ((int)blockIdx.x < wide_max / 4) tail_body<K, METHOD, 3>(a, P, pk, resident, wide_max); \
       }                                                                                        \
@@ -692,14 +693,14 @@ template <int METHOD>
 __global__ void __launch_bounds__(64 * 6) pte_batch_team_kernel(PteArgs a, MixParamsDev P,
                                                                 BatchArgs b) {
   extern __shared__ EosDev lds[];
-  const int nm = BinMaxNM(METHOD) - (int)blockIdx.y;
+  const int nm = b.max_nm - (int)blockIdx.y;
   const int claimed = min(b.bins[nm - 2].claimed, b.bins[nm - 2].records);
   int parked = 0;
   for (int k = 0; k < BATCH_BINS; ++k) parked += b.bins[k].claimed;
   if (parked > TEAM_MAX || (int)blockIdx.x >= claimed) return;
   stage_registry(lds, a.d_eos, a.nreg);
 #define SGM_ONE(K)                                                                             \
-  case K: team_body<K>(a, P, batch_park<K>(b)); break;
+  case K: team_body<K>(a, P, batch_park<METHOD, K>(b)); break;
   switch (nm) { SGM_ONE(2) SGM_ONE(3) SGM_ONE(4) SGM_ONE(5) SGM_ONE(6) }
 #undef SGM_ONE
 }
@@ -709,7 +710,7 @@ hipError_t batch_launch(const PteArgs &a, const MixParamsDev &P, const BatchArgs
                         const int *cells, const long *range, long n, int chunk, hipStream_t s) {
   const size_t lds = (size_t)a.nreg * sizeof(EosDev);
   const int ncu = device_cu_count();
-  const int nbin = BinMaxNM(METHOD) - 1;
+  const int nbin = b.max_nm - b.min_nm + 1;
   const long waves = (n + chunk - 1) / chunk;
   const int g = (int)(waves < 8L * ncu ? waves : 8L * ncu);
   pte_batch_bins_kernel<METHOD><<<dim3(g, nbin), 64, lds, s>>>(a, P, b, cells, range, chunk);

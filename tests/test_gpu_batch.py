@@ -337,3 +337,20 @@ def test_work_arrays_grow_with_headroom_and_are_given_back(sgm, workloads, torch
     call.run(ctx, 0)  # and the next call allocates again
     torch.cuda.synchronize()
     ctx.close()
+
+
+def test_plan_records_are_sized_by_their_bin(sgm, workloads, torch_gpu):
+    """A plan holds a straggler record per cell, (11 nm + 25) words of eight
+    bytes for nm materials, beside some 50 bytes a cell of lists and tables."""
+    torch = torch_gpu
+    ctx, _ = workloads.pool_context()
+    n = 1 << 18
+    call = Call(torch, sgm, workloads.uneven(ctx, n, seed=0x5EED0000 + 991), 0, True)
+    nm = (call.off[1:] - call.off[:-1]).cpu().numpy()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    p = PlanRun(sgm, ctx, call)
+    held = free - torch.cuda.mem_get_info()[0]
+    assert held < 8 * (11 * nm + 25).sum() + 50 * n + (16 << 20)
+    p.plan.close()
+    ctx.close()
