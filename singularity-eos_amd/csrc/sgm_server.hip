@@ -197,11 +197,18 @@ Layout make_layout(const sgm_server *sv, const std::vector<uint64_t> &ids) {
     L.st = take(8 * L.ncell);
     L.conv = take(4 * L.ncell);
     if (!sv->cfg.plain) {
-      // records for a twenty-second of the group's cells per material count
-      // (at least 776): a cell still iterating after the batch's threshold
-      // moves to its tail while records last, and keeps its lane past that
-      L.nrec = (int)std::max<long>(776, L.ncell / 22);
-      L.batch = take(batch_bytes(sv->cfg.method, L.ncell, L.nrec));
+      // records for a sixteenth of the group's cells per material count (at
+      // least 1024): a cell still iterating after the batch's threshold moves
+      // to its tail while records last, and keeps its lane past that. Groups
+      // whose cells need less with a record each (up to some 3,900) have that.
+      L.nrec = (int)std::max<long>(1024, L.ncell / 16);
+      size_t bytes = batch_bytes(sv->cfg.method, L.ncell, L.nrec);
+      const size_t each = batch_bytes(sv->cfg.method, L.ncell, 0);
+      if (each <= bytes) {
+        L.nrec = 0;
+        bytes = each;
+      }
+      L.batch = take(bytes);
     }
   }
   for (uint64_t t : ids) {

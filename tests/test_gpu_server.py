@@ -149,6 +149,24 @@ def test_request_larger_than_budget_is_refused(sgm, setup, torch_gpu):
     srv.close()
 
 
+@pytest.mark.parametrize("n", [1, 100, 3000, 20000])
+def test_working_set_follows_the_request(sgm, setup, torch_gpu, n):
+    """A closure request's share of the arena: about 0.9 KB a cell while every
+    cell has a straggler record (a one-cell request once took 2.8 MB), records
+    for a sixteenth of the cells per material count past that."""
+    ctx, w = setup
+    srv = sgm.Server(ctx, budget_bytes=64 << 20, params=sgm.mix_params(tight=True))
+    t, _ = submit(srv, w, ("pte", 0, n))
+    assert srv.wait(t)[0] == 0
+    peak = srv.stats()["arena_peak_bytes"]
+    srv.close()
+    nnz = int(w["offsets"][n])
+    # five doubles and an id per entry; 28 bytes of inputs and flags a cell, 24
+    # of keys and lists and the sort's copy of a key and a value (12)
+    state = 41 * nnz + 64 * n + (64 << 10)
+    assert peak <= state + min(740 * n, 2780 * max(1024, n // 16))
+
+
 def test_poisson_trace_completes(sgm, workloads, setup, torch_gpu):
     """A short open-loop trace through the load generator: every request
     completes and latencies are positive."""
