@@ -991,6 +991,8 @@ SGM_HD void fill_vinet(const EosDev &e, Real &rho, Real &temp, Real &sie, Real &
   }
   return;
 }
+// REC: on the table, fields come from the nodes' records (fill_from_records)
+template <bool REC>
 SGM_HD void fill_table(const EosDev &e, Real &rho, Real &temp, Real &sie, Real &press,
                      Real &cv, Real &bmod, unsigned long output, Lam &lam, int &err) {
   using namespace tq;
@@ -1030,14 +1032,8 @@ SGM_HD void fill_table(const EosDev &e, Real &rho, Real &temp, Real &sie, Real &
     lT = table::lT_(t, temp);
   }
   w = table::loc_rho_T(t, lRho, lT);
-#if defined(__HIP_DEVICE_COMPILE__)
-  const bool nodes = w == table::OnTable;
-#else
-  const bool nodes = false;
-#endif
-  if (nodes) {
-    // the four nodes' records, {sie, P} and {dEdT, bMod} apart (the vector
-    // FillEos was bound by the cache lines of its four separate fields)
+  if (REC && w == table::OnTable) {
+    // the four nodes' records, {sie, P} and {dEdT, bMod} apart
     const W1 wr = grid_weights(lRho, t.lRhoMin, t.dlRho, t.inv_dlRho, t.nRho);
     const W1 wt = grid_weights(lT, t.lTMin, t.dlT, t.inv_dlT, t.nT);
     const table::Pair2 *n0 = reinterpret_cast<const table::Pair2 *>(t.node) +
@@ -1076,11 +1072,23 @@ SGM_HD void base_fill(const EosDev &e, Real &rho, Real &temp, Real &sie, Real &p
   case KIND_STIFF: fill_gas(e, rho, temp, sie, press, cv, bmod, output, lam, err); return;
   case KIND_GRUN: fill_grun(e, rho, temp, sie, press, cv, bmod, output, lam, err); return;
   case KIND_VINET: fill_vinet(e, rho, temp, sie, press, cv, bmod, output, lam, err); return;
-  default: fill_table(e, rho, temp, sie, press, cv, bmod, output, lam, err); return;
+  default: fill_table<false>(e, rho, temp, sie, press, cv, bmod, output, lam, err); return;
   }
 }
+// Whether the vector FillEos on a table reads the nodes' records: for energy and
+// pressure, or three fields and more. It is bound by the cache lines it touches,
+// two a field, or two for all of a record's: four fields at 3,000,017 random
+// points 138 -> 94 us, energy and pressure 73 -> 69. Other pairs and single
+// fields read the fields' own arrays: the records' 4 MB fill an XCD's L2, where
+// one field's 1 MB leaves room (pressure 49 us, 69 from the records; heat
+// capacity and bulk modulus 75, 78; pressure and bulk modulus 73, 91).
+inline bool fill_from_records(unsigned long output) {
+  const unsigned long ep = tq::specific_internal_energy | tq::pressure,
+                      cb = tq::specific_heat | tq::bulk_modulus;
+  return (output & ep) == ep || ((output & cb) == cb && (output & ep) != 0);
+}
 // base_fill for a material known to be of kind KIND
-template <int KIND>
+template <int KIND, bool REC>
 SGM_HD void base_fill_k(const EosDev &e, Real &rho, Real &temp, Real &sie, Real &press, Real &cv,
                         Real &bmod, unsigned long output, Lam &lam, int &err) {
   if constexpr (KIND == KIND_IDEAL || KIND == KIND_STIFF)
@@ -1090,7 +1098,7 @@ SGM_HD void base_fill_k(const EosDev &e, Real &rho, Real &temp, Real &sie, Real 
   else if constexpr (KIND == KIND_VINET)
     fill_vinet(e, rho, temp, sie, press, cv, bmod, output, lam, err);
   else
-    fill_table(e, rho, temp, sie, press, cv, bmod, output, lam, err);
+    fill_table<REC>(e, rho, temp, sie, press, cv, bmod, output, lam, err);
 }
 
 // ---------------------------------------------------------------------------
@@ -1223,15 +1231,15 @@ SGM_HD void eos_rhoe_PT(const EosDev &e, Real P, Real T, Real &rho, Real &sie, L
 // shifted_eos.hpp:142-158): by the model's preferred input, (rho, T) or
 // (rho, sie); a modified IdealGas (whose preferred input is neither) is the
 // reference's EOS_ERROR, here ERRB_FILLEOS
-// eos_fill for a material of kind KIND (KIND < 0: any kind)
-template <int KIND>
+// eos_fill for a material of kind KIND (KIND < 0: any kind); REC: fill_table's
+template <int KIND, bool REC = false>
 SGM_HD void eos_fill_k(const EosDev &e, Real &rho, Real &temp, Real &sie, Real &press, Real &cv,
                        Real &bmod, unsigned long output, Lam &lam, int &err) {
   auto fill = [&](Real &r, Real &s) {
     if constexpr (KIND < 0)
       base_fill(e, r, temp, s, press, cv, bmod, output, lam, err);
     else
-      base_fill_k<KIND>(e, r, temp, s, press, cv, bmod, output, lam, err);
+      base_fill_k<KIND, REC>(e, r, temp, s, press, cv, bmod, output, lam, err);
   };
   if (!e.mods) {
     fill(rho, sie);

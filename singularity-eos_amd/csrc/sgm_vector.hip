@@ -96,7 +96,7 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-template <int KIND>
+template <int KIND, bool REC = false>
 __global__ void __launch_bounds__(256)
     fill_kernel(const EosDev *__restrict__ reg, int mat, double *rho, double *temp, double *sie,
                 double *press, double *cv, double *bmod, long n, unsigned long output,
@@ -127,7 +127,7 @@ __global__ void __launch_bounds__(256)
       lam.lT = lp[1];
     }
     int err = 0;
-    eos_fill_k<KIND>(ek, r, t, s, p, c, b, output, lam, err);
+    eos_fill_k<KIND, REC>(ek, r, t, s, p, c, b, output, lam, err);
     // an output set the model cannot fill (the reference's EOS_ERROR) writes
     // nothing: the point's arrays keep their values
     // (a modified material's FillEos may also change an input in place, as
@@ -262,7 +262,11 @@ hipError_t launch_fill(const EosDev &eh, const EosDev *d, int mat, double *rho, 
   case KIND_STIFF: fill_kernel<KIND_STIFF><<<g, 256, 0, s>>>(d, mat, rho, temp, sie, press, cv, bmod, n, output, ls, lam, errs); break;
   case KIND_GRUN: fill_kernel<KIND_GRUN><<<g, 256, 0, s>>>(d, mat, rho, temp, sie, press, cv, bmod, n, output, ls, lam, errs); break;
   case KIND_VINET: fill_kernel<KIND_VINET><<<g, 256, 0, s>>>(d, mat, rho, temp, sie, press, cv, bmod, n, output, ls, lam, errs); break;
-  default: fill_kernel<KIND_TABLE><<<g, 256, 0, s>>>(d, mat, rho, temp, sie, press, cv, bmod, n, output, ls, lam, errs); break;
+  default:
+    if (fill_from_records(output))
+      fill_kernel<KIND_TABLE, true><<<g, 256, 0, s>>>(d, mat, rho, temp, sie, press, cv, bmod, n, output, ls, lam, errs);
+    else
+      fill_kernel<KIND_TABLE><<<g, 256, 0, s>>>(d, mat, rho, temp, sie, press, cv, bmod, n, output, ls, lam, errs);
   }
   return hipGetLastError();
 }
