@@ -39,6 +39,24 @@ def run_plain(torch, ctx, a, method, params):
     return {k: v.cpu().numpy() for k, v in d.items()}
 
 
+def run_plain_kernels(torch, ctx, a, method, params):
+    """The per-call kernels whose loop runs every pass, which a call of uneven
+    cells takes while its stream is being captured (otherwise it runs as a
+    batch of the kernels that plans use)."""
+    d = dev(torch, a)
+    g, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s), torch.cuda.graph(g, stream=s):
+        rc = ctx.pte(method, a["ncell"], a["nnz"], d["offsets"], d["mat_ids"], d["rho"],
+                     d["vfrac"], d["sie"], d["temp"], d["press"], d["vfrac_tot"], d["sie_tot"],
+                     params=params, conv=d["conv"], niter=d["niter"], resid=d["resid"],
+                     err=d["err"], stream=s.cuda_stream)
+    assert rc == 0
+    g.replay()
+    torch.cuda.synchronize()
+    return {k: v.cpu().numpy() for k, v in d.items()}
+
+
 def run_batched(torch, sgm, ctx, a, method, params, autotune=False, replays=1):
     d = dev(torch, a)
     plan = sgm.Plan(ctx, a["ncell"], a["nnz"], d["offsets"], d["mat_ids"], method)
@@ -237,13 +255,14 @@ def test_empty_and_rejected_calls(sgm, pool, torch_gpu):
 
 def test_c2_full_size_invariants(sgm, workloads, pool, torch_gpu):
     """2^20 uneven cells at 1e-10 tolerance, batched path: conservation and
-    equilibrium properties that hold at any size, and batched == plain."""
+    equilibrium properties that hold at any size, and batched == the plain
+    kernels."""
     torch = torch_gpu
     ctx, _, _ = pool
     a = workloads.uneven(ctx, 1 << 20)
     params = sgm.mix_params(tight=True)
     b, _ = run_batched(torch, sgm, ctx, a, 0, params)
-    g = run_plain(torch, ctx, a, 0, params)
+    g = run_plain_kernels(torch, ctx, a, 0, params)
     assert_identical(b, g, "full size batched vs plain")
     off = a["offsets"]
     conv = b["conv"].astype(bool)
@@ -293,8 +312,8 @@ def test_straggler_parking_keeps_results(sgm, workloads, pool, torch_gpu, method
     iterations (so many that the tails' second level runs one lane per cell),
     after 20 (the default: the second level runs line-search groups) and 40,
     and with parking off, each output, flag and iteration count is
-    bit-identical to the plain per-call path, whose loop runs every pass (the
-    tails skip the passes of cells at a fixed point of the loop)."""
+    bit-identical to the plain per-call kernels, whose loop runs every pass
+    (the tails skip the passes of cells at a fixed point of the loop)."""
     torch = torch_gpu
     ctx, _, _ = pool
     a = workloads.uneven(ctx, 12000, seed=0x5EED0000 + 24)
@@ -304,7 +323,7 @@ def test_straggler_parking_keeps_results(sgm, workloads, pool, torch_gpu, method
     if method == 2:  # fixed temperature: each cell's first input temperature
         a["sie_tot"] = a["temp"][a["offsets"][:-1]].copy()
     params = sgm.mix_params(tight=method != 3)
-    g = run_plain(torch, ctx, a, method, params)
+    g = run_plain_kernels(torch, ctx, a, method, params)
     d = dev(torch, a)
     plan = sgm.Plan(ctx, a["ncell"], a["nnz"], d["offsets"], d["mat_ids"], method)
     for after in (2, 20, 40, 0, 1):
