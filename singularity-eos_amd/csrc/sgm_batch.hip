@@ -3,11 +3,11 @@
 // batched kernels (register-resident bins with straggler parking, tails),
 // bin bounds and record bases read on the device, so nothing comes back to
 // the host. The work arrays come from the context's batch workspaces, or from
-// the caller (the server's arena). What bounds a plain call over uneven cells is its slowest
-// cell's chain of Newton passes: the plain kernel runs it on one lane, behind
-// the wave's cells of other material counts and through every repeat of a
-// fixed point. 20,011 uneven cells, RhoT at 1e-10: 91 -> 12.2 ms; 1,000
-// cells 58 -> 2.7 ms; 3,001 cells PT 600 -> 147 ms.
+// the caller (the server's arena). What bounds a plain call over uneven cells
+// is its slowest cell's chain of Newton passes: the plain kernel runs it on one
+// lane, behind the wave's cells of other material counts and through every
+// repeat of a fixed point. 20,011 uneven cells, RhoT at 1e-10: 96 -> 8.3 ms; 200
+// cells 20 -> 1.5 ms; 3,001 cells PT 550 -> 88 ms.
 #include "sgm_internal.hpp"
 
 #include <hipcub/hipcub.hpp>

@@ -55,11 +55,13 @@ struct ParkArgs {
   const int *run_base = nullptr;    // per run: first record
   const int *run_cap = nullptr;     // per run: records available
   int *run_count = nullptr;         // per run: records claimed (claims past cap are not parked)
-  // per tail wave: its run (null, with wave_first: one run, wave w on the
-  // records of its w-th slot; nwaves is then an upper bound)
+  // per tail wave: its run. Null in a launch that bins share: one run, whose
+  // claimed records its tails divide among their waves (wave_first and nwaves
+  // unused)
   const int *wave_run = nullptr;
   const int *wave_first = nullptr;  // per tail wave: its first record within the run
   int nwaves = 0;
+  bool team = false;  // the parked cells are the team kernel's (PT)
   // the tail's second level: a cell still iterating `after2` iterations into
   // the first (one lane per cell) is saved again in its record for the
   // second, where TailGroup lanes share each cell
@@ -145,7 +147,7 @@ constexpr bool TailWide(int method, int nm) { return method == PTE_RHOT && nm >=
   hipError_t launch_pte_wave_##name(const PteArgs &a, const MixParamsDev &P, const int *cells, \
                                     long n, const long *range, hipStream_t s);                 \
   hipError_t launch_pte_bin_##name(int nm, const PteArgs &a, const MixParamsDev &P,            \
-                                   const int *cells, long n, const long *range, int *counter,  \
+                                   const int *cells, long n, int *counter,                     \
                                    int block, int cpw, int grid, const ParkArgs *park,         \
                                    hipStream_t s);                                             \
   hipError_t launch_pte_tail_##name(int nm, const PteArgs &a, const MixParamsDev &P,           \
@@ -214,19 +216,18 @@ inline hipError_t launch_pte_list(int method, const PteArgs &a, const MixParamsD
 // batched persistent bin (2..6 materials): cells all have nm materials
 inline hipError_t launch_pte_bin(int method, int nm, const PteArgs &a, const MixParamsDev &P,
                                  const int *cells, long n, int *counter, int block, int cpw,
-                                 int grid, hipStream_t s, const long *range = nullptr,
-                                 const ParkArgs *park = nullptr) {
+                                 int grid, hipStream_t s, const ParkArgs *park = nullptr) {
   switch (method) {
   case PTE_RHOT:
-    return launch_pte_bin_rhot(nm, a, P, cells, n, range, counter, block, cpw, grid, park, s);
+    return launch_pte_bin_rhot(nm, a, P, cells, n, counter, block, cpw, grid, park, s);
   case PTE_PT:
-    return launch_pte_bin_pt(nm, a, P, cells, n, range, counter, block, cpw, grid, park, s);
+    return launch_pte_bin_pt(nm, a, P, cells, n, counter, block, cpw, grid, park, s);
   case PTE_FIXED_T:
-    return launch_pte_bin_fixedt(nm, a, P, cells, n, range, counter, block, cpw, grid, park, s);
+    return launch_pte_bin_fixedt(nm, a, P, cells, n, counter, block, cpw, grid, park, s);
   case PTE_FIXED_P:
-    return launch_pte_bin_fixedp(nm, a, P, cells, n, range, counter, block, cpw, grid, park, s);
+    return launch_pte_bin_fixedp(nm, a, P, cells, n, counter, block, cpw, grid, park, s);
   case PTE_RHOU:
-    return launch_pte_bin_rhou(nm, a, P, cells, n, range, counter, block, cpw, grid, park, s);
+    return launch_pte_bin_rhou(nm, a, P, cells, n, counter, block, cpw, grid, park, s);
   default: return hipErrorInvalidValue;
   }
 }

@@ -266,7 +266,7 @@ hipError_t launch_one_bin(sgm_plan *p, size_t i, const PteArgs &a, const MixPara
   ParkArgs pk = b.park;
   pk.after = pk.rec ? p->park_after : 0;
   hipError_t e = launch_pte_bin(p->method, b.nm, a, P, cells, b.n, p->d_counters + i, b.block,
-                                b.cpw, b.grid, s, nullptr, &pk);
+                                b.cpw, b.grid, s, &pk);
   if (e != hipSuccess || pk.after <= 0) return e;
   return launch_pte_tail(p->method, b.nm, a, P, pk, s);
 }
@@ -377,7 +377,7 @@ hipError_t launch_bins(sgm_plan *p, const PteArgs &a, const MixParamsDev &P, hip
     ParkArgs pk = b.park;
     pk.after = pk.rec ? p->park_after : 0;
     if ((e = launch_pte_bin(p->method, b.nm, a, P, cells, b.n, p->d_counters + i, b.block,
-                            b.cpw, b.grid, s, nullptr, &pk)) != hipSuccess)
+                            b.cpw, b.grid, s, &pk)) != hipSuccess)
       return e;
     if (pk.after <= 0) continue;
     if (!fork) {
@@ -954,7 +954,7 @@ int sgm_plan_execute_bin(sgm_plan *p, int bin, double *rho, double *vfrac, doubl
     e = (b.nm < 2 || b.nm > 6)
             ? launch_list_bin(p, b, a, P, cells, s)
             : launch_pte_bin(p->method, b.nm, a, P, cells, b.n, p->d_counters + bin, b.block,
-                             b.cpw, b.grid, s, nullptr, &pk);
+                             b.cpw, b.grid, s, &pk);
   if (e == hipSuccess) e = hipEventRecord(ev[1], s);
   if (e == hipSuccess && pk.after > 0) e = launch_pte_tail(p->method, b.nm, a, P, pk, s);
   if (e == hipSuccess) e = hipEventRecord(ev[2], s);

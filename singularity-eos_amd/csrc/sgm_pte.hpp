@@ -2041,10 +2041,9 @@ SGM_HD void skip_to_last_pass(DriverState &d) {
 }
 
 // PTESolverPT for one cell on a team of NM waves, wave m holding material m: a
-// pass inverts each material's (P, T)
-// two times for the Jacobian and once per trial, 11 to 15 us each for a
-// Gruneisen, Vinet or table material on one wave, and the inversions of one
-// material start from its own last density only. So the materials' chains
+// pass inverts each material's (P, T) two times for the Jacobian and once per
+// trial, 8 to 11 us each for a Gruneisen, Vinet or table material on one wave,
+// and the inversions of one material start from its own last density only. So the materials' chains
 // run side by side on the CU's SIMDs, and every wave forms the sums from the
 // terms the team exchanges through LDS, in material order: the values and
 // the control flow are those of PtePT on every wave alike. Has the interface

@@ -2,9 +2,9 @@
 #include "sgm_pte_kernels.inl"
 namespace sgm {
 hipError_t launch_pte_bin_rhot(int nm, const PteArgs &a, const MixParamsDev &P, const int *cells,
-                             long n, const long *range, int *counter, int block, int cpw,
+                             long n, int *counter, int block, int cpw,
                              int grid, const ParkArgs *park, hipStream_t s) {
-  return kern::bin_launch<0>(nm, a, P, cells, n, counter, block, cpw, grid, s, range, park);
+  return kern::bin_launch<0>(nm, a, P, cells, n, counter, block, cpw, grid, s, park);
 }
 hipError_t launch_pte_tail_rhot(int nm, const PteArgs &a, const MixParamsDev &P,
                               const ParkArgs &park, hipStream_t s) {

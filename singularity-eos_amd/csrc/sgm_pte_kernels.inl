@@ -343,19 +343,17 @@ __attribute__((amdgpu_waves_per_eu(SGM_BIN_WAVES_PER_EU,
                                    SGM_BIN_WAVES_PER_EU))) pte_bin_kernel(PteArgs a, MixParamsDev P,
                                                       const int *__restrict__ cells,
                                                       long ncells, int *counter, int chunk,
-                                                      const long *range, ParkArgs pk) {
+                                                      ParkArgs pk) {
   extern __shared__ EosDev lds[];
   stage_registry(lds, a.d_eos, a.nreg);
-  if (range) {  // bin bounds computed on the device: {start, count} into cells
-    cells += range[0];
-    ncells = range[1];
-  }
   bin_body<NM, METHOD>(lds, a, P, cells, ncells, counter, chunk, pk);
 }
 
 // Resumes the parked cells of one bin in two levels. Level 1 (LEVEL 1): a
 // persistent grid of one-wave blocks walks the bin's tail wave slots (each
-// on records of a single signature run), one lane per cell; a cell that
+// on records of a single signature run; in a launch that the bins share the
+// bin's records are one run in claim order, divided over the grid), one lane
+// per cell; a cell that
 // reaches a fixed point of the Newton loop skips to its last pass, and a
 // cell still iterating pk.after2 iterations later is saved back into its
 // record for level 2 (finished cells clear their record's cell id). Level 2
@@ -377,8 +375,11 @@ constexpr int TailWavesL1() {
   return NM >= 5 ? SGM_TAIL_WAVES_PER_EU_LARGE : 2;
 }
 
-// Parked cells of a PT batch up to which each runs on a workgroup of its own
-// (four cells per CU)
+// Parked cells of a PT batch, over all its bins, up to which each runs on a
+// workgroup of its own (a wave per material): some four per CU of 256, sixteen
+// waves a CU on average. Past that one lane per cell has the higher throughput:
+// 400 parked cells (3,001 cells at default tolerances) 134 -> 95 ms, 2,700
+// parked cells 193 -> 225 ms.
 constexpr int TEAM_MAX = 1024;
 
 // Level 2 of a RhoT tail: the block's one wave takes record items (wave
@@ -473,7 +474,7 @@ __device__ __forceinline__ void tail_body(const PteArgs &a, const MixParamsDev &
     const int lpw = one_run && !grp
                         ? min(64, max(1, (claimed + (int)gridDim.x - 1) / (int)gridDim.x))
                         : per_slot;
-    if (METHOD == PTE_PT && one_run && pk.nwaves < 0) return;  // the team kernel's
+    if (pk.team) return;  // the team kernel's
     const long steps = !one_run ? (pk.nwaves + spb - 1) / spb : (claimed + lpw - 1) / lpw;
     for (long W = blockIdx.x; W < steps; W += gridDim.x) {
       int r = 0, i;
@@ -573,11 +574,9 @@ __device__ __forceinline__ ParkArgs batch_park(const BatchArgs &b) {
   pk.run_base = &t->first;
   pk.run_cap = &t->records;
   pk.run_count = &t->claimed;
-  // one run: its claimed records; -1 where the batch's parked cells go to the
-  // team kernel
   int parked = 0;
   for (int k = 0; k < BATCH_BINS; ++k) parked += b.bins[k].claimed;
-  pk.nwaves = parked <= TEAM_MAX ? -1 : 0;
+  pk.team = METHOD == PTE_PT && parked <= TEAM_MAX;
   pk.after2 = b.after2;
   pk.l2_count = &t->l2_count;
   pk.l2_next = &t->l2_next;
@@ -627,17 +626,17 @@ pte_batch_tails_kernel(PteArgs a, MixParamsDev P, BatchArgs b, int resident, int
 }
 
 // The parked cells of a PT bin, one per workgroup of NM waves (TeamPT), while
-// the batch parked at most TEAM_MAX; past that one lane per cell has the
-// higher throughput: 400 parked cells (3,001 cells at default tolerances) 134
-// -> 95 ms, 2,700 parked cells 193 -> 225 ms. Every wave of the team takes the same decisions: they follow
-// from values formed alike from the exchanged terms.
+// the batch parked at most TEAM_MAX. Every wave of the team takes the same
+// decisions: they follow from values formed alike from the exchanged terms.
 template <int NM>
 __device__ __forceinline__ void team_body(const PteArgs &a, const MixParamsDev &P,
                                           const ParkArgs &pk) {
   using Base = SysOf<NM, PTE_PT, false>;
   __shared__ typename TeamPT<NM>::Shared sh;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  if (wave >= NM) return;  // ended waves are not waited for
+  // the block has a wave for each of six materials: those past NM end here,
+  // and gfx950's barriers wait for the waves that have not ended only
+  if (wave >= NM) return;
   const int claimed = min(pk.run_count[0], pk.run_cap[0]);
   int turn = 0;
   for (int W = blockIdx.x; W < claimed; W += gridDim.x) {
@@ -771,8 +770,8 @@ hipError_t plain_launch(const PteArgs &a, const MixParamsDev &P, hipStream_t s) 
 template <int METHOD>
 hipError_t bin_launch(int nm, const PteArgs &a, const MixParamsDev &P, const int *cells, long n,
                       int *counter, int block, int cpw, int grid, hipStream_t s,
-                      const long *range = nullptr, const ParkArgs *park = nullptr) {
-  if (n <= 0 && !range) return hipSuccess;
+                      const ParkArgs *park = nullptr) {
+  if (n <= 0) return hipSuccess;
   const size_t lds = (size_t)a.nreg * sizeof(EosDev);
   const ParkArgs pk = park ? *park : ParkArgs{};
 #define SGM_BIN(K)                                                                             \
@@ -781,8 +780,7 @@ hipError_t bin_launch(int nm, const PteArgs &a, const MixParamsDev &P, const int
       static_assert(ParkWordCount<SysOf<K, METHOD, false>>() <= ParkStride(METHOD, K),         \
                     "park record");                                                            \
       if (pk.after > 0 && pk.stride < ParkStride(METHOD, K)) return hipErrorInvalidValue;      \
-      pte_bin_kernel<K, METHOD><<<grid, block, lds, s>>>(a, P, cells, n, counter, cpw, range,  \
-                                                         pk);                                  \
+      pte_bin_kernel<K, METHOD><<<grid, block, lds, s>>>(a, P, cells, n, counter, cpw, pk);    \
       break;                                                                                   \
     } else {                                                                                   \
       return hipErrorInvalidValue;                                                             \
@@ -811,7 +809,7 @@ hipError_t tail_launch(int nm, const PteArgs &a, const MixParamsDev &P, const Pa
   const int ncu = device_cu_count();
   const int cap = (nm >= 5 ? SGM_TAIL_WAVES_PER_EU_LARGE : 2) * 4 * ncu;
   const int G = TailGroup(METHOD, nm);
-  const int g1 = pk.wave_run ? (pk.nwaves + G - 1) / G : pk.nwaves * (64 / G);
+  const int g1 = (pk.nwaves + G - 1) / G;
   const int g = g1 < cap ? g1 : cap;
   const bool l2 = G > 1 && pk.after2 > 0 && pk.l2_count &&
                   P.line_search_max_iter <= G && (!TailWide(METHOD, nm) || pk.l2_next);
@@ -878,7 +876,6 @@ __global__ void __launch_bounds__(256) pte_list_kernel(PteArgs a, MixParamsDev P
     if (c < 0 || c >= a.ncell) continue;
     int off = 0;
     const int nm = cell_slice(a, c, off);
-    if (nm == 2 && a.skip_pairs) continue;
     switch (nm) {
     case 1: solve_cell_call<1, METHOD>(lds, a, P, c, off); break;
     case 2: solve_cell_call<2, METHOD>(lds, a, P, c, off); break;
