@@ -299,13 +299,12 @@ std::vector<size_t> bin_order(const sgm_plan *p) {
 // parked cells in claim order, the bins' own by signature: where the parked
 // cells outnumber the chip's waves and each pass is long, a wave of one
 // signature is the faster. PT 1,000 175 / 75 ms, 2^14 250 / 194, 2^15 246 / 211,
-// 2^16 249 / 261, 2^17 235 / 329; FixedP 2^16 46.7 / 37.3, 2^18 97 / 83,
-// 2^20 156 / 165.
+// 2^16 249 / 261, 2^17 235 / 329: apart past 2^15. FixedP 2^16 46.7 / 37.3, 2^18
+// 97 / 83, 2^20 156 / 165 (a third of those cells never converge), but the
+// 2^20 rho-P cells of get_sg_eos 140 / 67: together.
 bool shared_launch(const sgm_plan *p) {
-  const long most = p->method == PTE_PT        ? 1L << 15
-                    : p->method == PTE_FIXED_P ? 1L << 19
-                                               : 1L << 31;
-  return !p->own_shape && p->d_rec && p->method != PTE_RHOU && p->ncell <= most;
+  if (p->method == PTE_PT && p->ncell > 1L << 15) return false;
+  return !p->own_shape && p->d_rec && p->method != PTE_RHOU;
 }
 // Lanes of a wave that take cells: the cells of a plan spread over four waves
 // per CU; over one where each bin holds one signature, whose lanes run the same
