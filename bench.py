@@ -4,13 +4,14 @@ Headline (`value`): batched uneven closure — 2^20 mixed cells with 2..6
 materials from a pool of six (IdealGas x2, StiffGas, Gruneisen, Vinet, a
 Gruneisen-sampled rho-T table), PTESolverRhoT at the 1e-10 tolerances of
 singularity-eos/example/pte_2mat.cpp:169-180, FP64, one hipGraph launch per
-step (persistent kernel per material-count bin). A step restores the solver
+step (a persistent kernel that all material-count bins share, then their
+tails). A step restores the solver
 inputs (device-to-device copies; the closure works in place) and solves every
 cell; inputs are resident in HBM before timing starts.
 
 Reported beside it: the plain per-call path on the same cells and on the
 65,536-cell two-material closure, the 2^24-query table lookups, the
-roofline of the dominant bin kernel (HIP events on the launch stream) and the
+roofline of the closure kernels (HIP events on the launch stream) and the
 oracle CPU baseline on a bounded sample of the same workload.
 """
 import argparse
@@ -31,15 +32,14 @@ METRIC = "PTE closure cells/s at 1e-10 tol + p99 request latency, served vs plai
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
 
-# Per material-count bin of the headline workload, one execution of the bin's
-# kernels (pte_bin_kernel + both pte_tail_kernel levels): HBM bytes moved
-# (rocprofv3 FETCH_SIZE + WRITE_SIZE, scaled by the counters' reading of a
-# copy kernel of known size) and FP64 operations issued (SQ_INSTS_VALU_
-# {ADD,MUL,TRANS}_F64 x 64 lanes + FMA_F64 x 128). Measured with the
-# commands in profiles/pte_bins_uneven_2p20.md on the current kernels; None
-# where not measured.
-UNIT_HBM_BYTES = {2: 5.736e8, 3: 7.072e8, 4: 1.3336e9, 5: 2.3145e9, 6: 2.486e9}
-UNIT_FP64_OPS = {2: 1.137e10, 3: 2.156e10, 4: 1.969e10, 5: 1.984e10, 6: 1.655e10}
+# One execution of the headline workload's 2^20-cell plan (the shared bins kernel
+# and both tail levels): HBM bytes moved (rocprofv3 FETCH_SIZE + WRITE_SIZE,
+# scaled by the counters' reading of a copy kernel of known size) and FP64
+# operations issued (SQ_INSTS_VALU_{ADD,MUL,TRANS}_F64 x 64 lanes + FMA_F64 x
+# 128). Measured with the commands in profiles/shared_launch_counters.md.
+STEP_HBM_BYTES = 9.25e9
+STEP_FP64_OPS = 8.45e10
+STEP_CELLS = 1 << 20  # what they were measured on
 
 
 def log(*a):
@@ -290,7 +290,22 @@ def main():
     log(f"[bench] batched step times (ms): " + " ".join(f"{x:.1f}" for x in step_ms))
     step_stats = {"min": min(step_ms), "median": float(np.median(step_ms)), "max": max(step_ms)}
 
-    # per-bin kernel timing (HIP events on the launch stream)
+    # the closure of a step alone, without restoring the inputs
+    exec_ms = []
+    for _ in range(3):
+        restore()
+        e0, e1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        e0.record()
+        rc = plan.execute(work["rho"], work["vfrac"], work["sie"], work["temp"], work["press"], vt,
+                          st, params=params, conv=conv, niter=niter, stream=stream)
+        e1.record()
+        assert rc == 0, rc
+        torch.cuda.synchronize()
+        exec_ms.append(e0.elapsed_time(e1))
+    exec_ms = float(np.median(exec_ms))
+
+    # each bin's own kernels, one bin after another (HIP events on the launch
+    # stream): where the work is; the step runs the bins in a shared launch
     per_bin = []
     for bi, b in enumerate(bins):
         restore()
@@ -322,7 +337,10 @@ def main():
                             tail_kernel_ms=float(kms[1]), block=b["block"],
                             cells_per_wave=b["cells_per_wave"], grid=b["grid"],
                             tail_level2_cells=plan.tail_counts(stream=stream)[bi]))
-    extras = {"bins": per_bin, "step_ms": step_stats, "converged_frac": conv_frac,
+    extras = {"bins": per_bin,
+              "bins_note": "each bin by kernels of its own, one bin after another; a step "
+                           "launches the bins together",
+              "step_ms": step_stats, "converged_frac": conv_frac,
               "plan_build_ms": plan_build_ms,
               "plan_build_note": "sgm_plan_create for the 2^20-cell topology (bins, straggler "
                                  "records), measured once before the timed steps and not part "
@@ -606,39 +624,35 @@ def main():
                 f"{threads} threads, median of 3")
             log(f"[bench] get_sg_eos cpu: {nd / ddt:.4g} cells/s on {threads} threads")
 
-    # the dominant bin: its persistent kernel and its tail kernel together
-    # solve the bin's cells (a cell parked by the first finishes in the
-    # second), so the roofline is priced over the sum of their durations
-    dom = max(per_bin, key=lambda r: r["bulk_kernel_ms"] + r["tail_kernel_ms"])
-    nm = dom["nmat"] if dom["nmat"] else 4
-    kern_ms = dom["bulk_kernel_ms"] + dom["tail_kernel_ms"]
-    alg_bytes = dom["cells"] * bytes_per_cell(nm)
-    gbs = alg_bytes / (kern_ms * 1e-3) / 1e9
-    kname = f"pte_bin_kernel<{dom['nmat']}, 0> + pte_tail_kernel<{dom['nmat']}, 0> (RhoT)"
-    split = {"bulk_kernel_ms": dom["bulk_kernel_ms"], "tail_kernel_ms": dom["tail_kernel_ms"]}
-    traffic = UNIT_HBM_BYTES.get(nm)
+    # the closure kernels of a step: the bins' persistent kernel and the tails
+    # that finish the cells it parked
+    counts = {int(m): int(c) for m, c in zip(*np.unique(nm_cell, return_counts=True))}
+    alg_bytes = sum(c * bytes_per_cell(m) for m, c in counts.items())
+    gbs = alg_bytes / (exec_ms * 1e-3) / 1e9
+    kname = ("pte_batch_bins_kernel<0> + pte_batch_tails_kernel<0, 1> + "
+             "pte_batch_tails_kernel<0, 2> (RhoT, all bins)")
+    traffic = STEP_HBM_BYTES if n == STEP_CELLS else None
     hbm = {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
            "frac": gbs / HBM_PEAK_GBS, "traffic": traffic, "kernel": kname,
-           "bytes_per_cell": bytes_per_cell(nm)}
-    if flops_per_cell and nm in flops_per_cell:
-        tf = dom["cells"] * flops_per_cell[nm] / (kern_ms * 1e-3) / 1e12
+           "algorithmic_bytes": alg_bytes}
+    if flops_per_cell and all(m in flops_per_cell for m in counts):
+        flops = sum(c * flops_per_cell[m] for m, c in counts.items())
+        tf = flops / (exec_ms * 1e-3) / 1e12
         roofline = {"bound": "fp64_valu", "achieved": tf, "peak": FP64_PEAK_TFLOPS,
                     "unit": "TFLOP/s", "frac": tf / FP64_PEAK_TFLOPS, "traffic": traffic,
-                    "kernel": kname, "cells": dom["cells"], "ms": kern_ms, **split,
-                    "flops_per_cell": flops_per_cell[nm],
+                    "kernel": kname, "cells": n, "ms": exec_ms, "flops_per_cell": flops / n,
                     "algorithmic_bytes": alg_bytes,
-                    "pipe": "FP64 on the vector ALUs (no MFMA in this kernel); 78.6 TFLOP/s "
+                    "pipe": "FP64 on the vector ALUs (no MFMA in these kernels); 78.6 TFLOP/s "
                             "is MI355X's FP64 peak; achieved = the oracle's counted operations "
-                            "per cell (every +,-,*,/ and math call once) x cells / the bin's "
-                            "bulk + tail kernel time"}
-        ops = UNIT_FP64_OPS.get(nm)
-        if ops:
-            roofline["rocprof_fp64_TFLOPs"] = ops / (kern_ms * 1e-3) / 1e12
+                            "per cell (every +,-,*,/ and math call once) x cells / the time of "
+                            "one plan execution"}
+        if n == STEP_CELLS:
+            roofline["rocprof_fp64_TFLOPs"] = STEP_FP64_OPS / (exec_ms * 1e-3) / 1e12
             roofline["rocprof_fp64_frac"] = roofline["rocprof_fp64_TFLOPs"] / FP64_PEAK_TFLOPS
         extras["roofline_hbm"] = hbm
         extras["counted_flops_per_cell_by_nmat"] = flops_per_cell
     else:
-        roofline = dict(hbm, cells=dom["cells"], ms=kern_ms, **split)
+        roofline = dict(hbm, cells=n, ms=exec_ms)
 
     out = {
         "metric": METRIC, "value": cells_per_s, "unit": "cells/s", "n_gpus": 1,

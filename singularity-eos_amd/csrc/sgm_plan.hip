@@ -1,8 +1,9 @@
 // Batched PTE plan: bins the cells of one CSR topology by material count and
-// material signature (radix sort of a 64-bit key), picks a launch shape per
-// bin (optionally by timing candidates on the device: the autotuner), and
-// captures one hipGraph holding a counter reset plus one persistent kernel per
-// bin. Replays of the graph solve every cell with a single graph launch.
+// material signature (radix sort of a 64-bit key), and captures one hipGraph
+// holding a counter reset plus the kernels of all bins together or one
+// persistent kernel per bin (shared_launch), in default launch shapes or ones
+// that were set or timed on the device (the autotuner). Replays of the graph
+// solve every cell with a single graph launch.
 #include "sgm_internal.hpp"
 
 #include <hipcub/hipcub.hpp>
