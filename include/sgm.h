@@ -342,9 +342,10 @@ int sgm_driver_cache_info(sgm_ctx *ctx, long *out);
  * material count (2..6 run register-resident templated kernels; 2..4 for
  * RhoU; 9..64 one wave per cell) and by material signature and captures one
  * hipGraph whose persistent kernel nodes solve every bin: one node for all
- * register-resident bins, or one per bin (RhoU, large PT plans, and
- * after sgm_plan_set_shape or an autotuning that found it faster). method: 0 = RhoT, 1 = PT, 2 = FixedT, 3 = FixedP (the per-cell
- * sie_tot array of execute then holds the cell temperature / pressure, and
+ * register-resident bins, or one per bin (RhoU, few bins of many cells, and
+ * after sgm_plan_set_shape or an autotuning that found it faster).
+ * method: 0 = RhoT, 1 = PT, 2 = FixedT, 3 = FixedP (the per-cell sie_tot array
+ * of execute then holds the cell temperature / pressure, and
  * Tnorm is ignored), 4 = RhoU. Results are identical to sgm_pte_rhoT /
  * sgm_pte_PT / sgm_pte_fixedT / sgm_pte_fixedP / sgm_pte_rhoU on the same
  * inputs. The plan keeps device copies of offsets and mat_ids. */

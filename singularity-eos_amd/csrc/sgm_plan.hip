@@ -294,18 +294,40 @@ std::vector<size_t> bin_order(const sgm_plan *p) {
 // Whether a plan launches its bins together (one kernel for all bins, one per
 // tail level: launch_pte_batch_bins): unless a launch shape was set for one,
 // and not for RhoU, whose cells past four materials have no bin. The bins then
-// keep their own kernels, each bin's tail beside the next bins'. Apart against
-// together, uneven cells: RhoT 1,000 8.3 / 1.9 ms, 2^16 11.5 / 7.8, 2^20 21.3 /
-// 17.2; FixedT 2^14 4.9 / 3.6, 2^20 15.6 / 14.0. The shared tails take the
-// parked cells in claim order, the bins' own by signature: where the parked
-// cells outnumber the chip's waves and each pass is long, a wave of one
-// signature is the faster. PT 1,000 175 / 75 ms, 2^14 250 / 194, 2^15 246 / 211,
-// 2^16 249 / 261, 2^17 235 / 329: apart past 2^15. FixedP 2^16 46.7 / 37.3, 2^18
-// 97 / 83, 2^20 156 / 165 (a third of those cells never converge), but the
-// 2^20 rho-P cells of get_sg_eos 140 / 67: together.
+// keep their own kernels, each bin's tail beside the next bins'. Together, no
+// bin waits for another and small bins spread over more waves; apart, a bin has
+// a hardware queue while there are no more than four, and its tails take the
+// parked cells by signature instead of in claim order. So apart is the faster
+// for few bins of many cells, by method and number of bins past 2^limit cells
+// (0: always; 63: never). Apart / together in ms, uneven cells:
+//   RhoT    2 bins 1,000 4.0 / 3.2, 16,000 5.1 / 5.6, 250,000 8.3 / 9.0;
+//           3 bins 16,000 5.3 / 5.6, 250,000 10.3 / 9.3; 5 bins 2^20 21.3 / 17.2
+//   PT      1 bin (3 materials) 2,000 72 / 55, 8,000 59 / 136; 2 bins 4,000
+//           72 / 54, 16,000 63 / 120; 3 bins 4,000 122 / 72, 16,000 120 / 158;
+//           4 bins 16,000 184 / 185; 5 bins 2^14 250 / 194, 2^17 235 / 329
+//   FixedT  1 bin (5 materials) 2,000 3.2 / 3.1, 8,000 6.9 / 8.5; 2 bins 16,000
+//           1.6 / 1.5, 60,000 2.5 / 3.0; 3 bins 60,000 3.8 / 3.8, 250,000
+//           5.7 / 6.7; 5 bins 2^20 15.6 / 14.0
+//   FixedP  1 bin (2 materials) 500 3.7 / 4.3, 16,000 4.0 / 5.6; 2 bins 1,000
+//           7.4 / 8.7, 60,000 8.8 / 13.7; 3 bins 250,000 47 / 42; 5 bins 2^18
+//           97 / 83, the 2^20 rho-P cells of get_sg_eos 140 / 67
+// Bins of one signature each have no order to lose (4 gases a cell, RhoT, 2^17
+// cells 2.3 / 0.8 ms), but in PT their waves are too few to gain by it (2^14
+// pairs 0.29 / 0.31).
 bool shared_launch(const sgm_plan *p) {
-  if (p->method == PTE_PT && p->ncell > 1L << 15) return false;
-  return !p->own_shape && p->d_rec && p->method != PTE_RHOU;
+  if (p->own_shape || !p->d_rec || p->method == PTE_RHOU) return false;
+  constexpr int limit[4][5] = {
+      {12, 12, 63, 63, 63}, {11, 12, 13, 14, 15}, {12, 14, 16, 16, 63}, {0, 0, 63, 63, 63}};
+  int bins = 0;
+  long cells = 0;
+  for (const Bin &b : p->bins)
+    if (b.nruns > 0) {
+      ++bins;
+      cells += b.n;
+    }
+  if (p->nruns == bins && p->method != PTE_PT) return true;
+  const int l = limit[p->method][bins - 1];
+  return l > 0 && cells >> std::min(l, 62) == 0;
 }
 // Lanes of a wave that take cells: the cells of a plan spread over four waves
 // per CU; over one where each bin holds one signature, whose lanes run the same

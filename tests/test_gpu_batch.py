@@ -293,6 +293,17 @@ class PlanRun:
         return min(t[2:])
 
 
+def cells_of_counts(a, counts, n):
+    off = a["offsets"].astype(np.int64)
+    c = np.flatnonzero(np.isin(np.diff(off), counts))[:n]
+    assert len(c) == n
+    k = np.diff(off)[c]
+    new = np.concatenate([[0], np.cumsum(k)])
+    idx = np.repeat(off[c] - new[:-1], k) + np.arange(new[-1])
+    return dict({f: a[f][idx] for f in FIELDS + ("mat_ids",)}, offsets=new.astype(np.int32),
+                vfrac_tot=a["vfrac_tot"][c], sie_tot=a["sie_tot"][c], ncell=n, nnz=int(new[-1]))
+
+
 def pair_context(sgm, workloads):
     ctx = sgm.Context(2)
     ctx.set_ideal(0, *workloads.IDEAL_A)
@@ -304,7 +315,10 @@ def pair_context(sgm, workloads):
     ("pair", 0, 1 << 18, 1.25),   # 1.6 with the counters in one cache line
     ("pair", 0, 4096, 1.13),      # 1.2 with four lanes a wave
     ("uneven", 1, 1 << 17, 1.2),  # 1.5 with the tails in claim order
-    ("uneven", 0, 30011, 1.2), ("uneven", 2, 5003, 1.2), ("uneven", 3, 5003, 1.2)])
+    ("uneven", 0, 30011, 1.2), ("uneven", 2, 5003, 1.2), ("uneven", 3, 5003, 1.2),
+    # few bins of many cells, together in one launch: 2.1, 1.4, 1.9, 1.2, 1.45
+    ((3,), 1, 8000, 1.15), ((2,), 3, 8000, 1.15), ((2, 3), 1, 16000, 1.15),
+    ((5,), 2, 16000, 1.1), ((3,), 2, 30000, 1.15)])
 def test_default_schedule_keeps_pace(sgm, workloads, torch_gpu, pool, method, n, limit):
     """A plan's default schedule (mostly the launch that all its bins share)
     against a kernel per bin (a launch shape set, the default one): the same
@@ -315,7 +329,9 @@ def test_default_schedule_keeps_pace(sgm, workloads, torch_gpu, pool, method, n,
         a = workloads.pte2(n)
     else:
         ctx, _ = workloads.pool_context()
-        a = workloads.uneven(ctx, n, seed=0x5EED0000 + 960)
+        a = workloads.uneven(ctx, n if pool == "uneven" else 10 * n, seed=0x5EED0000 + 960)
+        if pool != "uneven":  # cells of these material counts only
+            a = cells_of_counts(a, pool, n)
     p = PlanRun(sgm, ctx, Call(torch, sgm, a, method, tight=pool == "uneven" and method == 0))
     default = p.run().result()
     default_ms = p.ms(torch)
