@@ -329,7 +329,8 @@ int sgm_get_sg_eos_noalloc(sgm_ctx *ctx, int nmat, int ncell, int cell_dim, int 
 /* No reference counterpart: frees the work buffers and the batched plan that
  * sgm_get_sg_eos keeps in the context between calls (for the 2^20-cell
  * uneven workload about 0.5 GB of straggler records plus the arenas), and the
- * work arrays of plain closure calls; the next calls rebuild them. This memory is outside any server's
+ * work arrays of plain closure calls (waiting for the last call that used them);
+ * the next calls rebuild them. This memory is outside any server's
  * hbm_budget_bytes. sgm_finalize releases it too. */
 int sgm_release_driver_cache(sgm_ctx *ctx);
 /* No reference counterpart: out[4] (HOST) = {calls that built the driver's
